@@ -343,10 +343,12 @@ double cyl_phi_scale(const fdmgpu_plan_t* P) {
 // Every stage addresses problem p of a batch at ptr + p * elems, or at tab[p]
 // when a device table of per-problem pointers is given (tab != null).
 using Tab = const void* const*;
-// Forward xy transforms: in (Tin) -> out (T).
+// Forward xy transforms: in (Tin) -> out (T).  reset (per problem, or null) is
+// set to 0 by the first launch (LaplCube and LaplRect only, not the streaming
+// plane kernels).
 template <typename Tin, typename T>
 int stage_fwd(fdmgpu_plan_t* P, const void* in, Tab in_tab, void* out, Tab out_tab, int count, hipStream_t s,
-              const int* done, int plane_class = FDMGPU_K_XY_FWD) {
+              const int* done, int plane_class = FDMGPU_K_XY_FWD, int* reset = nullptr) {
     const long elems = (long)P->nx * P->ny * P->nz;
     const double sx = P->dx * std::sqrt(2. / P->lx), sy = P->dy * std::sqrt(2. / P->ly);
     if (P->kind == 4) {   // LaplCyl3FFT2: phi (slowest axis) then z, as "y" passes
@@ -365,6 +367,7 @@ int stage_fwd(fdmgpu_plan_t* P, const void* in, Tab in_tab, void* out, Tab out_t
     if (P->kind == 3 && P->var.plane && P->logx == P->logy && plane_fits<T>(P->logx)) {
         PlaneArgs a{in, out, elems, elems, P->nz, count, sx, sy, P->tab_x, s, false, done, P->kfwd, in_tab, out_tab};
         a.stream_planes = P->var.plane == 2;
+        a.reset = reset;
         Timed tm(P, plane_class, s);
         HIPCHK((launch_plane<Tin, T, T>(P->logx, a)));
         return FDMGPU_OK;
@@ -373,6 +376,7 @@ int stage_fwd(fdmgpu_plan_t* P, const void* in, Tab in_tab, void* out, Tab out_t
         plane_rect_fits(P->logx, P->logy, sizeof(T) == 8)) {
         PlaneArgs a{in, out, elems, elems, P->nz, count, sx, sy, P->tab_x, s, false, done, P->kfwd, in_tab, out_tab};
         a.tables_y = P->tab_y;
+        a.reset = reset;
         Timed tm(P, plane_class, s);
         HIPCHK((launch_plane_rect<Tin, T, T>(P->logx, P->logy, a)));
         return FDMGPU_OK;
@@ -380,6 +384,7 @@ int stage_fwd(fdmgpu_plan_t* P, const void* in, Tab in_tab, void* out, Tab out_t
     if (P->kind == 3) {
         AxisArgs ax{in, out, (long)P->ny * P->nz, P->nx, P->nz, elems, elems, count, sx, P->tab_x, s, false, done,
                     P->kfwd, in_tab, out_tab, P->var.tile_x};
+        ax.reset = reset;
         {
             Timed tm(P, FDMGPU_K_X_TILE, s);
             HIPCHK((launch_xaxis<Tin, T, T>(P->logx, ax)));
@@ -393,6 +398,7 @@ int stage_fwd(fdmgpu_plan_t* P, const void* in, Tab in_tab, void* out, Tab out_t
     // rect: y (LaplRectFFT2: then x)
     AxisArgs ay{in, out, 0, P->nx, 1, elems, elems, count, sy, P->tab_y, s, false, done, P->kfwd, in_tab, out_tab,
                 P->var.tile_y};
+    ay.reset = reset;
     {
         Timed tm(P, FDMGPU_K_Y_TILE, s);
         HIPCHK((launch_yaxis<Tin, T, T>(P->logy, ay)));
@@ -643,7 +649,13 @@ int solve_refine(fdmgpu_plan_t* P, Work& W, double* ans, Tab ans_tab, const doub
         HIPCHK(hipMemcpyAsync(W.fcopy, rhs, bytes, hipMemcpyDeviceToDevice, s));
         rhs = W.fcopy;
     }
-    {
+    const bool fused = plane_capable(P) && square_planes(P) && P->var.plane && P->var.fuse;
+    // What the solve's first check finds in done[] and iters[]: with the separate
+    // residual, kernels before that check run without done[] (nothing has
+    // converged yet) and iters[], the check's counter, is zeroed by the first
+    // transform of a solve from zero, or by the caller, so the launch that
+    // clears both is left to the other paths.
+    if (P->periodic || fused || (first > 1 && !W.iters_zeroed)) {
         Timed tm(P, FDMGPU_K_OTHER, s);
         HIPCHK(launch_fill_int(W.done, W.iters, count, 0, s));
     }
@@ -672,7 +684,14 @@ int solve_refine(fdmgpu_plan_t* P, Work& W, double* ans, Tab ans_tab, const doub
     ra.stream = s;
     ra.f_tab = rhs_tab;
     ra.u_tab = ans_tab;
-    const bool fused = plane_capable(P) && square_planes(P) && P->var.plane && P->var.fuse;
+    ra.first_check = !fused;
+    auto done_now = [&]() -> const int* { return ra.first_check ? nullptr : W.done; };
+    auto check_residual = [&]() {
+        const hipError_t e = launch_residual(ra);
+        ra.base = ra.it;
+        ra.first_check = false;
+        return e;
+    };
     // u1 in FP32 scratch: separate-residual plane path (Dirichlet planes), solves 1 and 2 in
     // this call (the fused forward pass reads an FP32 iterate slower than it saves)
     const bool u1f = plane_capable(P) && P->var.plane && !fused && P->kinv == kDst && W.u32 && first == 1 &&
@@ -686,11 +705,12 @@ int solve_refine(fdmgpu_plan_t* P, Work& W, double* ans, Tab ans_tab, const doub
         ra.it = first - 1;
         ra.r32 = W.r32;
         Timed tm(P, FDMGPU_K_RESIDUAL_RHS, s);
-        HIPCHK(launch_residual(ra));
+        HIPCHK(check_residual());
     }
     for (int it = first; it <= last; ++it) {
         if (it == 1) {
-            rc = stage_fwd<double, float>(P, rhs, rhs_tab, W.r32, nullptr, count, s, W.done);
+            rc = stage_fwd<double, float>(P, rhs, rhs_tab, W.r32, nullptr, count, s, done_now(), FDMGPU_K_XY_FWD,
+                                          fused ? nullptr : W.iters);
         } else if (fused) {
             PlaneResidArgs pa{rhs, ans, W.r32, W.partial, elems, P->nz, count, ra.ix, ra.iy, ra.iz,
                               P->dx * std::sqrt(2. / P->lx), P->dy * std::sqrt(2. / P->ly), P->tab_x, s, W.done,
@@ -702,24 +722,25 @@ int solve_refine(fdmgpu_plan_t* P, Work& W, double* ans, Tab ans_tab, const doub
             if (it == 2 && first == 1) {   // the iterate after solve 1 was not certified
                 Timed tm(P, FDMGPU_K_RESIDUAL, s);
                 HIPCHK(launch_check(W.partial, P->nz, P->rtol, W.done, W.iters, W.resid, 1, count, s));
+                ra.base = 1;
             }
             rc = 0;
         } else {
             rc = stage_fwd<float, float>(P, W.r32, nullptr, W.r32, nullptr, count, s, W.done, FDMGPU_K_XY_FWD_R32);
         }
         if (rc) return rc;
-        rc = stage_tridiag<float>(P, W.r32, nullptr, count, s, W.done);
+        rc = stage_tridiag<float>(P, W.r32, nullptr, count, s, done_now());
         if (rc) return rc;
         if (u1f && it == 1)
-            rc = stage_inv<float, float>(P, W.r32, nullptr, W.u32, nullptr, count, s, false, W.done);
+            rc = stage_inv<float, float>(P, W.r32, nullptr, W.u32, nullptr, count, s, false, done_now());
         else
-            rc = stage_inv<float, double>(P, W.r32, nullptr, ans, ans_tab, count, s, it > 1, W.done,
+            rc = stage_inv<float, double>(P, W.r32, nullptr, ans, ans_tab, count, s, it > 1, done_now(),
                                           u1f && it == 2 ? W.u32 : nullptr);
         if (rc == -1) {   // rect accumulate
             dim3 g((unsigned)((elems + 255) / 256), count);
             Timed tm(P, FDMGPU_K_OTHER, s);
             hipLaunchKernelGGL(add_f32_to_f64, g, dim3(256), 0, s, BatchPtr<double>{ans, ans_tab, elems},
-                               (const float*)W.r32, elems, elems, (const int*)W.done);
+                               (const float*)W.r32, elems, elems, done_now());
             HIPCHK(hipGetLastError());
             rc = 0;
         }
@@ -732,7 +753,7 @@ int solve_refine(fdmgpu_plan_t* P, Work& W, double* ans, Tab ans_tab, const doub
         ra.u_f32 = u1f && it == 1;
         ra.bad = it == last ? W.bad : nullptr;
         Timed tm(P, ra.r32 ? FDMGPU_K_RESIDUAL_RHS : FDMGPU_K_RESIDUAL, s);
-        HIPCHK(launch_residual(ra));
+        HIPCHK(check_residual());
     }
     return FDMGPU_OK;
 }

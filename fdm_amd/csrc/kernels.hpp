@@ -115,6 +115,7 @@ struct PlaneArgs {
                                   // problems flagged done get out = base
     bool stream_planes = false;   // plane_stream_kernel: FP64, N = 128, plain (no accum / base / done)
     const void* tables_y = nullptr;   // rectangular planes: the y axis's DST tables (tables: x)
+    int* reset = nullptr;         // per batch item: set to 0 by the launch (one-plane-per-block kernels), or null
 };
 
 struct AxisArgs {
@@ -133,6 +134,7 @@ struct AxisArgs {
     const void* const* in_tab;
     const void* const* out_tab;
     int tile;             // pencils per block (16/32/64; 0 = default_tile)
+    int* reset = nullptr; // per batch item: set to 0 by the launch, or null
 };
 
 struct ZcrArgs {

@@ -212,9 +212,12 @@ __global__ __launch_bounds__(kTileX * kTileY) void ns_fgh_kernel(Grid g, Fields 
 
 // Poisson right-hand side with the pressure boundary values moved over
 // (src/ns_cube.cpp:204-235); interior i, k, j in [1, n]
-__global__ __launch_bounds__(kTileX * kTileY) void ns_rhs_kernel(Grid g, Fields f, const TileGrid tg) {
+__global__ __launch_bounds__(kTileX * kTileY) void ns_rhs_kernel(Grid g, Fields f, const TileGrid tg,
+                                                                    int* __restrict__ iters) {
     int bx, by, bz;
     if (!xcd_tile(tg, bx, by, bz)) return;
+    // the warm-started refinement's check counter (Work::iters_zeroed)
+    if (iters && blockIdx.x == 0 && threadIdx.x == 0 && threadIdx.y == 0) *iters = 0;
     const int j = bx * kTileX + (int)threadIdx.x + 1;
     const int k = tile_row(by) + 1;
     const int i = bz + 1;
@@ -356,8 +359,6 @@ int ns_enqueue_step(fdmgpu_ns_t* N, hipStream_t s, hipEvent_t* ev = nullptr) {
     hipLaunchKernelGGL(ns_fgh_kernel, dim3(tf.blocks()), b2, 0, s, g, N->f, tf);
     NS_HIPCHK(hipGetLastError());
     NS_HIPCHK(mark(2));
-    hipLaunchKernelGGL(ns_rhs_kernel, dim3(ti.blocks()), b2, 0, s, g, N->f, ti);
-    NS_HIPCHK(hipGetLastError());
     // FP32+refine: from the second step on, x still holds the previous step's
     // pressure, a close iterate for the new right-hand side; the refinement
     // continues from it (FP64 residual, then FP32 corrections: inner solves
@@ -366,6 +367,9 @@ int ns_enqueue_step(fdmgpu_ns_t* N, hipStream_t s, hipEvent_t* ev = nullptr) {
     // those of a cold solve.
     const bool refine = N->plan->precision == FDMGPU_F32_REFINE64;
     const bool warm = refine && N->warm_ok;
+    hipLaunchKernelGGL(ns_rhs_kernel, dim3(ti.blocks()), b2, 0, s, g, N->f, ti, warm ? N->plan->w.iters : nullptr);
+    NS_HIPCHK(hipGetLastError());
+    N->plan->w.iters_zeroed = warm;
     // a projection that misses the tolerance marks the run: the solve's final
     // norm check sets d_bad on the device (no host round trip, no extra
     // launch); only this step's solves carry the flag
@@ -374,6 +378,7 @@ int ns_enqueue_step(fdmgpu_ns_t* N, hipStream_t s, hipEvent_t* ev = nullptr) {
                                      std::max(2, N->plan->max_iter - 1))
                   : plan_solve(N->plan, N->plan->w, N->f.x, nullptr, N->f.RHS, nullptr, 1, s);
     N->plan->w.bad = nullptr;
+    N->plan->w.iters_zeroed = false;
     if (rc) return rc;
     NS_HIPCHK(mark(3));
     hipLaunchKernelGGL(ns_update_kernel, dim3(ti.blocks()), b2, 0, s, g, N->f, ti);

@@ -26,6 +26,7 @@ struct Work {
     double* fcopy = nullptr;            // f kept when a refine solve runs in place
     size_t fcopy_bytes = 0;
     int* bad = nullptr;                 // device flag set when a solve ends above tolerance (or null)
+    bool iters_zeroed = false;          // the caller's own kernel zeroes iters[] before a solve with first > 1
 };
 
 using Tab = const void* const*;

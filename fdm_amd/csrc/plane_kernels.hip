@@ -111,7 +111,7 @@ template <typename Tin, typename Tout, typename T, int LOGN, int ACC, int KIND>
 __global__ __launch_bounds__(PlaneCfg<LOGN>::NT)
 __attribute__((amdgpu_waves_per_eu(PlaneCfg<LOGN>::template waves<T>()))) void plane_dst_kernel(
     const BatchPtr<const Tin> in, const BatchPtr<Tout> out, const T sx, const T sy, const T* __restrict__ tables,
-    const int* __restrict__ done, const float* __restrict__ base, const long base_bs) {
+    const int* __restrict__ done, const float* __restrict__ base, const long base_bs, int* __restrict__ reset) {
     using C = PlaneCfg<LOGN>;
     using S = DstShape<LOGN>;
     using IO = PencilIO<KIND, LOGN>;
@@ -172,6 +172,8 @@ __attribute__((amdgpu_waves_per_eu(PlaneCfg<LOGN>::template waves<T>()))) void p
             else dst[y * n + x] = (Tout)v;
         });
     }
+    // (at the end: a store ahead of the plane's loads stands in their order)
+    if (reset && blockIdx.x == 0 && tid == 0) reset[blockIdx.y] = 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -615,7 +617,7 @@ static hipError_t plane_k(const PlaneArgs& a) {
     const BatchPtr<const Tin> in{(const Tin*)a.in, a.in_tab, a.bs_in};
     const BatchPtr<Tout> out{(Tout*)a.out, a.out_tab, a.bs_out};
     hipLaunchKernelGGL(k, dim3(a.nplanes, a.batch), dim3(C::NT), lds, a.stream, in, out, (T)a.sx, (T)a.sy,
-                       (const T*)a.tables, a.done, a.base, a.bs_out);
+                       (const T*)a.tables, a.done, a.base, a.bs_out, a.reset);
     return hipGetLastError();
 }
 

@@ -52,7 +52,8 @@ template <typename Tin, typename Tout, typename T, int LXN, int LYN, int ACC>
 __global__ __launch_bounds__((RectCfg<LXN, LYN>::NT))
 __attribute__((amdgpu_waves_per_eu(RectCfg<LXN, LYN>::template waves<T>()))) void plane_rect_kernel(
     const BatchPtr<const Tin> in, const BatchPtr<Tout> out, const T sx, const T sy, const T* __restrict__ tab_x,
-    const T* __restrict__ tab_y, const int* __restrict__ done, const float* __restrict__ base, const long base_bs) {
+    const T* __restrict__ tab_y, const int* __restrict__ done, const float* __restrict__ base, const long base_bs,
+    int* __restrict__ reset) {
     using C = RectCfg<LXN, LYN>;
     using SX = typename C::SX;
     using SY = typename C::SY;
@@ -121,6 +122,8 @@ __attribute__((amdgpu_waves_per_eu(RectCfg<LXN, LYN>::template waves<T>()))) voi
             else dst[y * nx + x] = (Tout)v;
         });
     }
+    // (at the end: a store ahead of the plane's loads stands in their order)
+    if (reset && blockIdx.x == 0 && tid == 0) reset[blockIdx.y] = 0;
 }
 
 template <typename Tin, typename Tout, typename T, int LXN, int LYN, int ACC>
@@ -133,7 +136,7 @@ static hipError_t rect_k(const PlaneArgs& a) {
     const BatchPtr<const Tin> in{(const Tin*)a.in, a.in_tab, a.bs_in};
     const BatchPtr<Tout> out{(Tout*)a.out, a.out_tab, a.bs_out};
     hipLaunchKernelGGL(k, dim3(a.nplanes, a.batch), dim3(C::NT), lds, a.stream, in, out, (T)a.sx, (T)a.sy,
-                       (const T*)a.tables, (const T*)a.tables_y, a.done, a.base, a.bs_out);
+                       (const T*)a.tables, (const T*)a.tables_y, a.done, a.base, a.bs_out, a.reset);
     return hipGetLastError();
 }
 

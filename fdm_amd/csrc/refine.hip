@@ -37,6 +37,117 @@ __device__ __forceinline__ void block_sum2(double& a, double& b, double* sh) {
     b = sh[kResBlock];
 }
 
+
+// ---------------------------------------------------------------------------
+// The convergence check rides on the residual launch: a block stores its norm
+// partials, counts itself, and the problem's last block sums all of them and
+// sets the flag.  A check kernel of its own cost 4.6 us and a gap before it
+// after every residual, 9 us at 255^3, and needed a launch that cleared the
+// flags first.  With the fold a residual launch ends about 5 us later and five
+// launches of a solve are gone: 255^3 526 -> 507 us a solve, 32 x 127^3 1320 ->
+// 1310, 512 uneven problems 3797 -> 3680, a 127^3 cavity step 203 -> 199.
+// What makes the fold cheap is that no release fence is needed: the partials
+// are the only data handed over, and they are stored and loaded as agent-scope
+// atomics, which go past the XCD's L2 by themselves.  (A release at agent scope
+// writes the XCD's whole L2 back; with one per block the residual launch took
+// twice its time.)  The storing wave waits until its stores are complete before
+// it counts, so whoever reads the last count reads every partial.
+// The counter is the problem's iters[] entry: it enters the launch at `base`
+// (0, or the iteration the problem's previous check wrote) and leaves it as `it`.
+// ---------------------------------------------------------------------------
+constexpr int kCheckBlock = 1024;   // threads the summation order is written for
+constexpr int kCheckUnroll = 8;
+
+struct CheckArgs {
+    double tol;
+    int* done;
+    int* iters;
+    double* resid;
+    int* bad;
+    int it, base;
+};
+
+__device__ __forceinline__ void put_partial(double* __restrict__ slot, const double rr, const double ff) {
+    __hip_atomic_store(slot, rr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(slot + 1, ff, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// True in every thread of the problem's last block.  Wave 0 has stored the
+// block's partials (put_partial); all threads call this.
+__device__ __forceinline__ bool last_block(int* __restrict__ count, const int base, const int nblocks) {
+    __shared__ int last;
+    if (threadIdx.x == 0) {
+        asm volatile("" ::: "memory");
+        wait_vmem_all();   // the partials are where every XCD reads them
+        asm volatile("" ::: "memory");
+        const int old = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = old == base + nblocks - 1;
+    }
+    __syncthreads();
+    return last != 0;
+}
+
+// Fixed-order sum of problem p's nblk partials and its verdict, by the NT
+// threads of one block: kCheckBlock virtual threads add partials t, t +
+// kCheckBlock, ... with kCheckUnroll loads in flight, then the sums of 64
+// virtual threads are added in order.  The order depends on nblk only, not on
+// the batch or on NT.
+// bad (the final certification of a solve, or null): set to 1 when a problem
+// checked here ends above the tolerance (or its residual is NaN).
+template <int NT>
+__device__ void norm_verdict(double* partial, const int p, const int nblk, const CheckArgs& k) {
+    __shared__ double sh[2 * (kCheckBlock / 64)];
+    double* const part = partial + (long)p * nblk * 2;
+    auto get = [&](int i) { return __hip_atomic_load(part + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    for (int vw = (int)(threadIdx.x >> 6); vw < kCheckBlock / 64; vw += NT / 64) {
+        const int vt = vw * 64 + (int)(threadIdx.x & 63);
+        double rr = 0.0, ff = 0.0;
+        for (int b = 0; b < nblk; b += kCheckBlock * kCheckUnroll) {
+            double vr[kCheckUnroll], vf[kCheckUnroll];
+#pragma unroll
+            for (int j = 0; j < kCheckUnroll; ++j) {
+                if (b + j * kCheckBlock >= nblk) {   // the same for every thread
+                    vr[j] = 0.0;
+                    vf[j] = 0.0;
+                    continue;
+                }
+                const int i = b + j * kCheckBlock + vt;
+                const int ic = i < nblk ? i : nblk - 1;   // clamped: no branch around the loads
+                const double x = get(2 * ic), y = get(2 * ic + 1);
+                vr[j] = i < nblk ? x : 0.0;
+                vf[j] = i < nblk ? y : 0.0;
+            }
+#pragma unroll
+            for (int j = 0; j < kCheckUnroll; ++j) {
+                rr += vr[j];
+                ff += vf[j];
+            }
+        }
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            rr += __shfl_xor(rr, d, 64);
+            ff += __shfl_xor(ff, d, 64);
+        }
+        if ((threadIdx.x & 63) == 0) {
+            sh[2 * vw] = rr;
+            sh[2 * vw + 1] = ff;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double a = 0.0, c = 0.0;
+        for (int i = 0; i < kCheckBlock / 64; ++i) {
+            a += sh[2 * i];
+            c += sh[2 * i + 1];
+        }
+        const double rel = c > 0.0 ? sqrt(a / c) : sqrt(a);
+        k.resid[p] = rel;
+        k.iters[p] = k.it;
+        k.done[p] = rel <= k.tol ? 1 : 0;
+        if (!(rel <= k.tol) && k.bad) k.bad[0] = 1;
+    }
+}
+
 // r = f - A u (FP64), r32 = (float) r; partial[p][c] = (sum r^2, sum f^2)
 // over chunk c of problem blockIdx.y.  A chunk is a contiguous range of rows
 // (row = z * ny + y), one wave per row and the lanes along x.  The gridDim.x
@@ -49,7 +160,7 @@ __global__ __launch_bounds__(kResBlock) void residual_kernel(
     const BatchPtr<const double> f, const BatchPtr<const double> u, float* __restrict__ r32,
     double* __restrict__ partial, const int nx, const int ny, const int nz, const double ix, const double iy,
     const double iz, const double* __restrict__ sy, const double* __restrict__ lx,
-    const double* __restrict__ ux, const long bs, const int* __restrict__ done) {
+    const double* __restrict__ ux, const long bs, const int* __restrict__ done, const CheckArgs check) {
     __shared__ double sh[2 * kResBlock];
     const int p = blockIdx.y;
     if (done && done[p]) return;
@@ -91,10 +202,8 @@ __global__ __launch_bounds__(kResBlock) void residual_kernel(
         }
     }
     block_sum2<double>(rr, ff, sh);
-    if (threadIdx.x == 0) {
-        partial[((long)p * nblk + c) * 2 + 0] = rr;
-        partial[((long)p * nblk + c) * 2 + 1] = ff;
-    }
+    if (threadIdx.x == 0) put_partial(partial + ((long)p * nblk + c) * 2, rr, ff);
+    if (last_block(check.iters + p, check.base, nblk)) norm_verdict<kResBlock>(partial, p, nblk, check);
 }
 
 // 3-D residual: a block of TX x TY threads owns the tile x in [x0, x0+TX),
@@ -108,10 +217,11 @@ __global__ __launch_bounds__(kResBlock) void residual_kernel(
 // Blocks go round-robin over the 8 XCDs; the logical block index (problem,
 // chunk, tile) is dealt out in contiguous slabs per XCD, so neighbouring
 // tiles, whose halo rows overlap, share an L2.
-// Norm partials: one per (z-granule of kZGran planes, tile, wave), written by
-// the wave that covers it: partial[p][(g * tiles + tile) * NW + w].  The
-// chunk length (a whole number of granules, chosen per launch to fill the
-// GPU) changes neither the layout nor the summation order.
+// Norm partials: one per (z-granule of kZGran planes, tile), the sum of the
+// waves' sums in a fixed order: partial[p][g * tiles + tile].  The chunk length
+// (a whole number of granules, chosen per launch to fill the GPU) changes
+// neither the layout nor the summation order.  (One per wave was 16 times as
+// many for the last block to read: 512 KB at 255^3.)
 constexpr int kZGran = 8;
 constexpr int kXcdCount = 8;
 
@@ -129,9 +239,12 @@ template <int TX, int TY, bool WRITE, typename Tu>
 __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(8))) void residual_tile_kernel(
     const BatchPtr<const double> f, const BatchPtr<const Tu> u, float* __restrict__ r32,
     double* __restrict__ partial, const int nx, const int ny, const int nz, const double ix, const double iy,
-    const double iz, const long bs, const int batch, const int chunk_gran, const int* __restrict__ done) {
+    const double iz, const long bs, const int batch, const int chunk_gran, const int* __restrict__ done,
+    const CheckArgs check) {
     constexpr int NT = TX * TY, NW = NT / 64;
+    static_assert(NW == 16 && NT == kCheckBlock, "16 wave sums per granule");
     __shared__ double t[2][TY + 2][TX + 2];
+    __shared__ double wsum[2][2 * NW];   // the waves' (rr, ff) of a granule, by the granule's parity
     const int gtx = (nx + TX - 1) / TX, gty = (ny + TY - 1) / TY;
     const int ngran = (nz + kZGran - 1) / kZGran, zc = (ngran + chunk_gran - 1) / chunk_gran;
     const int tiles = gtx * gty, per_problem = tiles * zc;
@@ -219,6 +332,26 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(8))) voi
     });
     double um = uval(um0, z0 - 1), uc = uval(uc0, z0);
     double rr = 0.0, ff = 0.0;
+    // Granule g's wave sums (in LDS behind a barrier) added up by wave 0, whose
+    // lane g - g0 keeps them to the end of the chunk: at most 64 granules, as
+    // nz <= 511.  (Stored as they come, in the loop, they cost 25 us of 60 at
+    // 255^3: a store past the L2 stands in the order of the wave's loads.)
+    const int g0 = z0 / kZGran;
+    double keep_r = 0.0, keep_f = 0.0;
+    auto flush = [&](const int g) {
+        if (threadIdx.x >= 64) return;
+        const int l = (int)threadIdx.x & (NW - 1);
+        double a = wsum[g & 1][2 * l], b = wsum[g & 1][2 * l + 1];
+#pragma unroll
+        for (int d = NW / 2; d > 0; d >>= 1) {
+            a += __shfl_xor(a, d, 64);
+            b += __shfl_xor(b, d, 64);
+        }
+        if ((int)threadIdx.x == g - g0) {
+            keep_r = a;
+            keep_f = b;
+        }
+    };
     __syncthreads();
     // one plane: `cur` holds u at z+1, f and halos at z; the next D-1 sets are
     // in flight; `fre` is refilled for D planes later
@@ -229,6 +362,7 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(8))) voi
         if (hOK) b[hr][hcol] = (double)cur.h;
         load_slot(fre, z + D + 1, z + D);   // in flight while planes z .. z+D-1 are computed
         __syncthreads();   // b complete; the other buffer's readers (plane z-1) are past this point
+        if ((z & (kZGran - 1)) == 0 && z != z0) flush(z / kZGran - 1);
         const double udn = uval(cur.u, z + 1);
         const double fv = cur.f;
         const double au = (b[ty + 1][tx] - 2.0 * uc + b[ty + 1][tx + 2]) * ix +
@@ -239,16 +373,15 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(8))) voi
             ff += fv * fv;
             if constexpr (WRITE) r32[p * bs + o + c0] = (float)r;
         }
-        if ((z & (kZGran - 1)) == kZGran - 1 || z + 1 == nz) {   // granule done: the wave's partial
+        if ((z & (kZGran - 1)) == kZGran - 1 || z + 1 == nz) {   // granule done: the wave's sums
 #pragma unroll
             for (int d = 32; d > 0; d >>= 1) {
                 rr += __shfl_xor(rr, d, 64);
                 ff += __shfl_xor(ff, d, 64);
             }
             if ((threadIdx.x & 63) == 0) {
-                const long slot = ((long)p * ngran * tiles + (long)(z / kZGran) * tiles + tile) * NW + (threadIdx.x >> 6);
-                partial[slot * 2 + 0] = rr;
-                partial[slot * 2 + 1] = ff;
+                wsum[(z / kZGran) & 1][2 * (threadIdx.x >> 6)] = rr;
+                wsum[(z / kZGran) & 1][2 * (threadIdx.x >> 6) + 1] = ff;
             }
             rr = 0.0;
             ff = 0.0;
@@ -266,6 +399,12 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(8))) voi
         constexpr int q = decltype(kk)::value;
         if (z + q < z1) step(z + q, sl[q], sl[(q + D) % NS]);
     });
+    __syncthreads();
+    flush((z1 - 1) / kZGran);
+    if (threadIdx.x < 64 && g0 + (int)threadIdx.x <= (z1 - 1) / kZGran)
+        put_partial(partial + ((long)p * ngran * tiles + (long)(g0 + (int)threadIdx.x) * tiles + tile) * 2, keep_r,
+                    keep_f);
+    if (last_block(check.iters + p, check.base, per_problem)) norm_verdict<NT>(partial, p, ngran * tiles, check);
 }
 
 // z-chunk length in granules: whole columns unless the batch is too small to
@@ -281,7 +420,7 @@ static int res_chunk_gran(int nx, int ny, int nz, int batch, int tiles) {
 
 template <int TX, int TY, typename Tu>
 static void launch_residual_tile(const ResidualArgs& a, const BatchPtr<const double>& f,
-                                 const BatchPtr<const Tu>& u) {
+                                 const BatchPtr<const Tu>& u, const CheckArgs& check) {
     const int tiles = ((a.nx + TX - 1) / TX) * ((a.ny + TY - 1) / TY);
     const int cg = res_chunk_gran(a.nx, a.ny, a.nz, a.batch, tiles);
     const int ngran = (a.nz + kZGran - 1) / kZGran, zc = (ngran + cg - 1) / cg;
@@ -290,69 +429,20 @@ static void launch_residual_tile(const ResidualArgs& a, const BatchPtr<const dou
     const dim3 grid((unsigned)((total + kXcdCount - 1) / kXcdCount * kXcdCount));
     if (a.r32)
         hipLaunchKernelGGL((residual_tile_kernel<TX, TY, true, Tu>), grid, dim3(TX * TY), 0, a.stream, f, u, a.r32,
-                           a.partial, a.nx, a.ny, a.nz, a.ix, a.iy, a.iz, a.bs, a.batch, cg, a.done);
+                           a.partial, a.nx, a.ny, a.nz, a.ix, a.iy, a.iz, a.bs, a.batch, cg,
+                           a.first_check ? nullptr : a.done, check);
     else
         hipLaunchKernelGGL((residual_tile_kernel<TX, TY, false, Tu>), grid, dim3(TX * TY), 0, a.stream, f, u, a.r32,
-                           a.partial, a.nx, a.ny, a.nz, a.ix, a.iy, a.iz, a.bs, a.batch, cg, a.done);
+                           a.partial, a.nx, a.ny, a.nz, a.ix, a.iy, a.iz, a.bs, a.batch, cg,
+                           a.first_check ? nullptr : a.done, check);
 }
 
-// One block per problem: fixed-order sum of the partials, then the flag.  A
-// thread adds partials tid, tid + kCheckBlock, ... with kCheckUnroll loads in
-// flight (a 255^3 problem has 32768 partials), then the waves' sums are added
-// in wave order; the order depends on nblk only, not on the batch.
-constexpr int kCheckBlock = 1024;
-constexpr int kCheckUnroll = 8;
-
-// bad (the final certification of a solve, or null): set to 1 when a
-// problem checked here ends above the tolerance (or its residual is NaN).
-__global__ __launch_bounds__(kCheckBlock) void check_kernel(const double* __restrict__ partial, const int nblk,
-                                                           const double tol, int* __restrict__ done,
-                                                           int* __restrict__ iters, double* __restrict__ resid,
-                                                           const int it, int* __restrict__ bad) {
-    __shared__ double sh[2 * (kCheckBlock / 64)];
-    const int p = blockIdx.x;
-    if (done[p]) return;
-    const auto part = as_global(partial + (long)p * nblk * 2);
-    double rr = 0.0, ff = 0.0;
-    for (int b = 0; b < nblk; b += kCheckBlock * kCheckUnroll) {
-        double vr[kCheckUnroll], vf[kCheckUnroll];
-#pragma unroll
-        for (int k = 0; k < kCheckUnroll; ++k) {
-            const int i = b + k * kCheckBlock + (int)threadIdx.x;
-            const int ic = i < nblk ? i : nblk - 1;   // clamped: no branch around the loads
-            const double x = part[2 * ic], y = part[2 * ic + 1];
-            vr[k] = i < nblk ? x : 0.0;
-            vf[k] = i < nblk ? y : 0.0;
-        }
-#pragma unroll
-        for (int k = 0; k < kCheckUnroll; ++k) {
-            rr += vr[k];
-            ff += vf[k];
-        }
-    }
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) {
-        rr += __shfl_xor(rr, d, 64);
-        ff += __shfl_xor(ff, d, 64);
-    }
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-        sh[2 * w] = rr;
-        sh[2 * w + 1] = ff;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double a = 0.0, c = 0.0;
-        for (int i = 0; i < kCheckBlock / 64; ++i) {
-            a += sh[2 * i];
-            c += sh[2 * i + 1];
-        }
-        const double rel = c > 0.0 ? sqrt(a / c) : sqrt(a);
-        resid[p] = rel;
-        iters[p] = it;
-        if (rel <= tol) done[p] = 1;
-        else if (bad) bad[0] = 1;
-    }
+// The check as a launch of its own, one block per problem: after the fused
+// plane transform and the periodic residual.
+__global__ __launch_bounds__(kCheckBlock) void check_kernel(double* __restrict__ partial, const int nblk,
+                                                           const CheckArgs k) {
+    if (k.done[blockIdx.x]) return;
+    norm_verdict<kCheckBlock>(partial, (int)blockIdx.x, nblk, k);
 }
 
 __global__ void fill_int_kernel(int* __restrict__ a, int* __restrict__ b, const int n, const int v) {
@@ -366,46 +456,46 @@ __global__ void fill_int_kernel(int* __restrict__ a, int* __restrict__ b, const 
 constexpr long kResMaxBlocks = 1024;   // per problem
 
 hipError_t launch_residual(const ResidualArgs& a) {
-    const unsigned nblk = (unsigned)residual_partials(a.nx, a.ny, a.nz, a.nz > 1 || a.three);
-    dim3 grid(nblk, a.batch);
+    const CheckArgs check{a.tol, a.done, a.iters, a.resid, a.bad, a.it, a.base};
+    const int* const skip = a.first_check ? nullptr : a.done;
     const BatchPtr<const double> f{a.f, a.f_tab, a.bs}, u{a.u, a.u_tab, a.bs};
     if (a.nz > 1 || a.three) {
         const ResTile t = res_tile(a.nx);
         if (a.u_f32) {
             const BatchPtr<const float> u32{(const float*)a.u, a.u_tab, a.bs};
-            if (t.tx == 32) launch_residual_tile<32, 32>(a, f, u32);
-            else if (t.tx == 64) launch_residual_tile<64, 16>(a, f, u32);
-            else launch_residual_tile<128, 8>(a, f, u32);
+            if (t.tx == 32) launch_residual_tile<32, 32>(a, f, u32, check);
+            else if (t.tx == 64) launch_residual_tile<64, 16>(a, f, u32, check);
+            else launch_residual_tile<128, 8>(a, f, u32, check);
         } else {
-            if (t.tx == 32) launch_residual_tile<32, 32>(a, f, u);
-            else if (t.tx == 64) launch_residual_tile<64, 16>(a, f, u);
-            else launch_residual_tile<128, 8>(a, f, u);
+            if (t.tx == 32) launch_residual_tile<32, 32>(a, f, u, check);
+            else if (t.tx == 64) launch_residual_tile<64, 16>(a, f, u, check);
+            else launch_residual_tile<128, 8>(a, f, u, check);
         }
     } else if (a.u_f32) {
         return hipErrorInvalidValue;
-    } else if (a.sy) {
-        hipLaunchKernelGGL((residual_kernel<false, true>), grid, dim3(kResBlock), 0, a.stream, f, u, a.r32,
-                           a.partial, a.nx, a.ny, 1, a.ix, a.iy, 0.0, a.sy, a.lx, a.ux, a.bs, a.done);
     } else {
-        hipLaunchKernelGGL((residual_kernel<false, false>), grid, dim3(kResBlock), 0, a.stream, f, u, a.r32,
-                           a.partial, a.nx, a.ny, 1, a.ix, a.iy, 0.0, nullptr, nullptr, nullptr, a.bs, a.done);
+        const dim3 grid((unsigned)residual_partials(a.nx, a.ny, a.nz, false), a.batch);
+        if (a.sy)
+            hipLaunchKernelGGL((residual_kernel<false, true>), grid, dim3(kResBlock), 0, a.stream, f, u, a.r32,
+                               a.partial, a.nx, a.ny, 1, a.ix, a.iy, 0.0, a.sy, a.lx, a.ux, a.bs, skip, check);
+        else
+            hipLaunchKernelGGL((residual_kernel<false, false>), grid, dim3(kResBlock), 0, a.stream, f, u, a.r32,
+                               a.partial, a.nx, a.ny, 1, a.ix, a.iy, 0.0, nullptr, nullptr, nullptr, a.bs, skip,
+                               check);
     }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(check_kernel, dim3(a.batch), dim3(kCheckBlock), 0, a.stream, a.partial, (int)nblk, a.tol, a.done,
-                       a.iters, a.resid, a.it, a.bad);
     return hipGetLastError();
 }
 
-hipError_t launch_check(const double* partial, int nblk, double tol, int* done, int* iters, double* resid, int it,
-                        int batch, hipStream_t s) {
-    hipLaunchKernelGGL(check_kernel, dim3(batch), dim3(kCheckBlock), 0, s, partial, nblk, tol, done, iters, resid, it,
-                       (int*)nullptr);
+hipError_t launch_check(double* partial, int nblk, double tol, int* done, int* iters, double* resid, int it, int batch,
+                        hipStream_t s) {
+    hipLaunchKernelGGL(check_kernel, dim3(batch), dim3(kCheckBlock), 0, s, partial, nblk,
+                       CheckArgs{tol, done, iters, resid, nullptr, it, 0});
     return hipGetLastError();
 }
 
-// partials per problem: 3-D, one per (z-granule, tile, wave) of
-// residual_tile_kernel; 2-D, chunks of about 4 rows, a multiple of 8 (one
+// partials per problem the scratch holds: 3-D, one per (z-granule, tile, wave)
+// of residual_tile_kernel's tiling (it writes one per granule and tile; the
+// periodic residual takes as many chunks); 2-D, chunks of about 4 rows, a multiple of 8 (one
 // slab per XCD), at most kResMaxBlocks
 long residual_partials(int nx, int ny, int nz, bool three) {
     if (three) {
@@ -562,8 +652,8 @@ hipError_t launch_periodic_residual(const PeriodicResidualArgs& a) {
                        a.done);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !a.check) return e;
-    hipLaunchKernelGGL(check_kernel, dim3(a.batch), dim3(kCheckBlock), 0, a.stream, (const double*)a.partial, a.nblk,
-                       a.tol, a.done, a.iters, a.resid, a.it, a.bad);
+    hipLaunchKernelGGL(check_kernel, dim3(a.batch), dim3(kCheckBlock), 0, a.stream, a.partial, a.nblk,
+                       CheckArgs{a.tol, a.done, a.iters, a.resid, a.bad, a.it, 0});
     return hipGetLastError();
 }
 

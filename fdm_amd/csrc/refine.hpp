@@ -30,12 +30,16 @@ struct ResidualArgs {
     const void* const* u_tab;
     bool u_f32 = false;         // u holds FP32 values (3-D only)
     int* bad = nullptr;         // final certification: set to 1 when a problem ends above tol
+    int base = 0;               // iters[] as the launch finds it (0, or the previous check's iteration)
+    bool first_check = false;   // the solve's first check: done[] is not read, only set
 };
 
+// The residual, its norms and the convergence check, in one launch.  iters[]
+// of every problem not done holds `base`.
 hipError_t launch_residual(const ResidualArgs& a);
 // norm check over `nblk` partials per problem (fixed order); see refine.hip
-hipError_t launch_check(const double* partial, int nblk, double tol, int* done, int* iters, double* resid, int it,
-                        int batch, hipStream_t s);
+hipError_t launch_check(double* partial, int nblk, double tol, int* done, int* iters, double* resid, int it, int batch,
+                        hipStream_t s);
 // partials per problem of launch_residual (three: the 7-point cube operator)
 long residual_partials(int nx, int ny, int nz, bool three);
 // a[i] = b[i] = v for i < n (b may be null); a kernel, so it can be captured in a graph
