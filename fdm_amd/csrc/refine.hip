@@ -52,9 +52,15 @@ __device__ __forceinline__ void block_sum2(double& a, double& b, double* sh) {
 // writes the XCD's whole L2 back; with one per block the residual launch took
 // twice its time.)  The storing wave waits until its stores are complete before
 // it counts, so whoever reads the last count reads every partial.
+// Storing, counting and reading back are three round trips past the L2, about
+// 4 us of a block's life.  One round of blocks (kFoldBlocks) hides that at its
+// end; with more rounds each pays it, and a check of its own is cheaper: 50
+// problems of 511 x 71 points, 6400 blocks of four rows, took 467 us a solve
+// folded and 332 apart.
 // The counter is the problem's iters[] entry: it enters the launch at `base`
 // (0, or the iteration the problem's previous check wrote) and leaves it as `it`.
 // ---------------------------------------------------------------------------
+constexpr long kFoldBlocks = 1024;   // blocks of a residual launch that checks itself, at most
 constexpr int kCheckBlock = 1024;   // threads the summation order is written for
 constexpr int kCheckUnroll = 8;
 
@@ -65,6 +71,8 @@ struct CheckArgs {
     double* resid;
     int* bad;
     int it, base;
+    bool fold;    // the residual's last block checks (else check_kernel, a launch of its own)
+    bool first;   // check_kernel: every problem, whatever done[] holds
 };
 
 __device__ __forceinline__ void put_partial(double* __restrict__ slot, const double rr, const double ff) {
@@ -203,6 +211,7 @@ __global__ __launch_bounds__(kResBlock) void residual_kernel(
     }
     block_sum2<double>(rr, ff, sh);
     if (threadIdx.x == 0) put_partial(partial + ((long)p * nblk + c) * 2, rr, ff);
+    if (!check.fold) return;
     if (last_block(check.iters + p, check.base, nblk)) norm_verdict<kResBlock>(partial, p, nblk, check);
 }
 
@@ -404,6 +413,7 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(8))) voi
     if (threadIdx.x < 64 && g0 + (int)threadIdx.x <= (z1 - 1) / kZGran)
         put_partial(partial + ((long)p * ngran * tiles + (long)(g0 + (int)threadIdx.x) * tiles + tile) * 2, keep_r,
                     keep_f);
+    if (!check.fold) return;
     if (last_block(check.iters + p, check.base, per_problem)) norm_verdict<NT>(partial, p, ngran * tiles, check);
 }
 
@@ -420,13 +430,14 @@ static int res_chunk_gran(int nx, int ny, int nz, int batch, int tiles) {
 
 template <int TX, int TY, typename Tu>
 static void launch_residual_tile(const ResidualArgs& a, const BatchPtr<const double>& f,
-                                 const BatchPtr<const Tu>& u, const CheckArgs& check) {
+                                 const BatchPtr<const Tu>& u, CheckArgs& check) {
     const int tiles = ((a.nx + TX - 1) / TX) * ((a.ny + TY - 1) / TY);
     const int cg = res_chunk_gran(a.nx, a.ny, a.nz, a.batch, tiles);
     const int ngran = (a.nz + kZGran - 1) / kZGran, zc = (ngran + cg - 1) / cg;
     // the kernel re-deals the blocks (problem, chunk, tile) to XCD slabs
     const long total = (long)tiles * zc * a.batch;
     const dim3 grid((unsigned)((total + kXcdCount - 1) / kXcdCount * kXcdCount));
+    check.fold = total <= kFoldBlocks;
     if (a.r32)
         hipLaunchKernelGGL((residual_tile_kernel<TX, TY, true, Tu>), grid, dim3(TX * TY), 0, a.stream, f, u, a.r32,
                            a.partial, a.nx, a.ny, a.nz, a.ix, a.iy, a.iz, a.bs, a.batch, cg,
@@ -438,10 +449,10 @@ static void launch_residual_tile(const ResidualArgs& a, const BatchPtr<const dou
 }
 
 // The check as a launch of its own, one block per problem: after the fused
-// plane transform and the periodic residual.
+// plane transform, the periodic residual and residuals of many blocks.
 __global__ __launch_bounds__(kCheckBlock) void check_kernel(double* __restrict__ partial, const int nblk,
                                                            const CheckArgs k) {
-    if (k.done[blockIdx.x]) return;
+    if (!k.first && k.done[blockIdx.x]) return;
     norm_verdict<kCheckBlock>(partial, (int)blockIdx.x, nblk, k);
 }
 
@@ -456,11 +467,13 @@ __global__ void fill_int_kernel(int* __restrict__ a, int* __restrict__ b, const 
 constexpr long kResMaxBlocks = 1024;   // per problem
 
 hipError_t launch_residual(const ResidualArgs& a) {
-    const CheckArgs check{a.tol, a.done, a.iters, a.resid, a.bad, a.it, a.base};
+    long nblk = 0;
+    CheckArgs check{a.tol, a.done, a.iters, a.resid, a.bad, a.it, a.base, true, a.first_check};
     const int* const skip = a.first_check ? nullptr : a.done;
     const BatchPtr<const double> f{a.f, a.f_tab, a.bs}, u{a.u, a.u_tab, a.bs};
     if (a.nz > 1 || a.three) {
         const ResTile t = res_tile(a.nx);
+        nblk = (long)((a.nx + t.tx - 1) / t.tx) * ((a.ny + t.ty - 1) / t.ty) * ((a.nz + kZGran - 1) / kZGran);
         if (a.u_f32) {
             const BatchPtr<const float> u32{(const float*)a.u, a.u_tab, a.bs};
             if (t.tx == 32) launch_residual_tile<32, 32>(a, f, u32, check);
@@ -474,7 +487,9 @@ hipError_t launch_residual(const ResidualArgs& a) {
     } else if (a.u_f32) {
         return hipErrorInvalidValue;
     } else {
-        const dim3 grid((unsigned)residual_partials(a.nx, a.ny, a.nz, false), a.batch);
+        nblk = residual_partials(a.nx, a.ny, a.nz, false);
+        const dim3 grid((unsigned)nblk, a.batch);
+        check.fold = nblk * a.batch <= kFoldBlocks;
         if (a.sy)
             hipLaunchKernelGGL((residual_kernel<false, true>), grid, dim3(kResBlock), 0, a.stream, f, u, a.r32,
                                a.partial, a.nx, a.ny, 1, a.ix, a.iy, 0.0, a.sy, a.lx, a.ux, a.bs, skip, check);
@@ -483,13 +498,16 @@ hipError_t launch_residual(const ResidualArgs& a) {
                                a.partial, a.nx, a.ny, 1, a.ix, a.iy, 0.0, nullptr, nullptr, nullptr, a.bs, skip,
                                check);
     }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || check.fold) return e;
+    hipLaunchKernelGGL(check_kernel, dim3(a.batch), dim3(kCheckBlock), 0, a.stream, a.partial, (int)nblk, check);
     return hipGetLastError();
 }
 
 hipError_t launch_check(double* partial, int nblk, double tol, int* done, int* iters, double* resid, int it, int batch,
                         hipStream_t s) {
     hipLaunchKernelGGL(check_kernel, dim3(batch), dim3(kCheckBlock), 0, s, partial, nblk,
-                       CheckArgs{tol, done, iters, resid, nullptr, it, 0});
+                       CheckArgs{tol, done, iters, resid, nullptr, it, 0, false, false});
     return hipGetLastError();
 }
 
@@ -653,7 +671,7 @@ hipError_t launch_periodic_residual(const PeriodicResidualArgs& a) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !a.check) return e;
     hipLaunchKernelGGL(check_kernel, dim3(a.batch), dim3(kCheckBlock), 0, a.stream, a.partial, a.nblk,
-                       CheckArgs{a.tol, a.done, a.iters, a.resid, a.bad, a.it, 0});
+                       CheckArgs{a.tol, a.done, a.iters, a.resid, a.bad, a.it, 0, false, false});
     return hipGetLastError();
 }
 
