@@ -55,31 +55,51 @@ constexpr double cos32(int m) {
 }
 constexpr double sin32(int m) { return cos32(m - 8); }
 
-// (re, im) *= exp(-2 pi i K / L), L | 32, all compile time.
+// Butterfly (a, b) <- (a + w b, a - w b), w = exp(-2 pi i K / L), L | 32, all
+// compile time.  Every product feeds an explicit fma (6 operations where w is
+// neither 1 nor -i, 8 as a product and two sums), which also leaves the
+// compiler no choice of which product to contract: the same transform gives the
+// same bits in every kernel.
 template <int L, int K, typename T>
-__device__ __forceinline__ void twiddle_ct(T& re, T& im) {
-    constexpr int k = ((K % L) + L) % L;
-    if constexpr (k == 0) {
-    } else if constexpr (4 * k == L) {   // * (-i)
-        T t = re;
-        re = im;
-        im = -t;
-    } else if constexpr (2 * k == L) {
-        re = -re;
-        im = -im;
-    } else if constexpr (4 * k == 3 * L) {   // * (+i)
-        T t = re;
-        re = -im;
-        im = t;
+__device__ __forceinline__ void butterfly(T& ar, T& ai, T& br, T& bi) {
+    static_assert(0 <= K && 2 * K < L, "first half turn");
+    if constexpr (K == 0) {
+        const T r = ar - br, i = ai - bi;
+        ar += br;
+        ai += bi;
+        br = r;
+        bi = i;
+    } else if constexpr (4 * K == L) {   // w = -i
+        const T r = ar - bi, i = ai + br;
+        ar += bi;
+        ai -= br;
+        br = r;
+        bi = i;
+    } else if constexpr (8 * K == L || 8 * K == 3 * L) {   // w = +-sqrt(1/2) - i sqrt(1/2)
+        constexpr T h = (T)kQuarter[4];
+        const T d = 8 * K == L ? br + bi : bi - br, e = 8 * K == L ? bi - br : -(br + bi);
+        br = fma(-h, d, ar);
+        bi = fma(-h, e, ai);
+        ar = fma(h, d, ar);
+        ai = fma(h, e, ai);
     } else {
-        constexpr int m = k * (32 / L);
+        constexpr int m = K * (32 / L);
         constexpr T c = (T)cos32(m);
         constexpr T s = (T)(-sin32(m));
-        T r = re * c - im * s;
-        T i = re * s + im * c;
-        re = r;
-        im = i;
+        const T r = fma(-s, bi, fma(c, br, ar)), i = fma(c, bi, fma(s, br, ai));
+        br = fma(T(2), ar, -r);
+        bi = fma(T(2), ai, -i);
+        ar = r;
+        ai = i;
     }
+}
+
+// (re, im) *= c + i s
+template <typename T>
+__device__ __forceinline__ void rotate(T& re, T& im, const T c, const T s) {
+    const T r = fma(-s, im, c * re), i = fma(c, im, s * re);
+    re = r;
+    im = i;
 }
 
 // In-register forward DFT of size R (natural order in and out).
@@ -106,12 +126,7 @@ __device__ __forceinline__ void dft(T (&re)[R], T (&im)[R]) {
                 static_for<0, len / 2>([&](auto kk) {
                     constexpr int a = decltype(bb)::value * len + decltype(kk)::value;
                     constexpr int b = a + len / 2;
-                    T tr = re[b], ti = im[b];
-                    twiddle_ct<len, decltype(kk)::value>(tr, ti);
-                    re[b] = re[a] - tr;
-                    im[b] = im[a] - ti;
-                    re[a] = re[a] + tr;
-                    im[a] = im[a] + ti;
+                    butterfly<len, decltype(kk)::value>(re[a], im[a], re[b], im[b]);
                 });
             });
         });
@@ -166,6 +181,10 @@ struct DstLane {
         }
     }
     __device__ __forceinline__ T sine(const int j2) const { return sp[j2]; }
+    __device__ __forceinline__ void twiddle(const int k2, T& c, T& s) const {
+        c = twr[k2];
+        s = twi[k2];
+    }
 };
 
 // The same constants with the shifted sines read from a per-block LDS copy of
@@ -191,6 +210,38 @@ struct DstLaneLdsSine {
         for (int m = tid; m < S::N; m += nt) lds_sines[m] = tables[2 * S::N + m];
     }
     __device__ __forceinline__ T sine(const int j2) const { return sl[S::N1 * j2]; }
+    __device__ __forceinline__ void twiddle(const int k2, T& c, T& s) const {
+        c = twr[k2];
+        s = twi[k2];
+    }
+};
+
+// All the constants from LDS: the shifted sines as above, the twiddles from a
+// copy laid out [k2][t] as (re, im) pairs, so a job's lanes read consecutive
+// pairs.  For kernels that hold data in registers through a pass.
+template <typename T, int LOGN>
+struct DstLaneLds {
+    using S = DstShape<LOGN>;
+    static constexpr int kValues = S::N + 2 * S::N1 * S::N2;   // values of T in LDS (8-byte aligned for float)
+    const T* sl;
+    const T* tl;
+    __device__ __forceinline__ void init(const T* lds, const int t) {
+        sl = lds + t;
+        tl = lds + S::N + 2 * t;
+    }
+    __device__ static void fill(const T* __restrict__ tables, T* lds, const int tid, const int nt) {
+        for (int m = tid; m < S::N; m += nt) lds[m] = tables[2 * S::N + m];
+        for (int m = tid; m < S::N1 * S::N2; m += nt) {
+            const int k2 = m / S::N1, t = m % S::N1;
+            lds[S::N + 2 * m] = tables[t * k2];
+            lds[S::N + 2 * m + 1] = tables[S::N + t * k2];
+        }
+    }
+    __device__ __forceinline__ T sine(const int j2) const { return sl[S::N1 * j2]; }
+    __device__ __forceinline__ void twiddle(const int k2, T& c, T& s) const {
+        c = tl[2 * S::N1 * k2];
+        s = tl[2 * S::N1 * k2 + 1];
+    }
 };
 
 // LDS layouts of a set of pencils.  Measured on gfx950: b32 accesses and b64
@@ -431,11 +482,9 @@ __device__ __forceinline__ void pencil_pairs(T* __restrict__ lds, const Lane& L,
             dft<N2>(yr, yi);
 #pragma unroll
             for (int k2 = 1; k2 < N2; ++k2) {
-                const T c = L.twr[k2], s = L.twi[k2];
-                const T r = yr[k2] * c - yi[k2] * s;
-                const T i = yr[k2] * s + yi[k2] * c;
-                yr[k2] = r;
-                yi[k2] = i;
+                T c, s;
+                L.twiddle(k2, c, s);
+                rotate(yr[k2], yi[k2], c, s);
             }
             wave_lds_sync();
 #pragma unroll
@@ -635,11 +684,9 @@ __device__ __forceinline__ void dst_pairs128(T* __restrict__ lds, const Lane& L,
     dft<N2>(yr, yi);
 #pragma unroll
     for (int k2 = 1; k2 < N2; ++k2) {
-        const T c = L.twr[k2], s = L.twi[k2];
-        const T r = yr[k2] * c - yi[k2] * s;
-        const T i = yr[k2] * s + yi[k2] * c;
-        yr[k2] = r;
-        yi[k2] = i;
+        T c, s;
+        L.twiddle(k2, c, s);
+        rotate(yr[k2], yi[k2], c, s);
     }
     wave_lds_sync();
 #pragma unroll
