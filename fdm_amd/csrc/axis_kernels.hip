@@ -108,11 +108,13 @@ __device__ __forceinline__ void xtile_sweep(const int xb, const bool on, LD&& ld
 }
 
 // rows = nrows pencils of IO::n points (N-1 Dirichlet, N periodic), contiguous;
-// batch via blockIdx.y.
+// batch via blockIdx.y.  tiles_pp > 0: tiles_pp tiles per plane of rows_pp rows,
+// so a tile's rows (and the pencils that share a transform) lie in one plane.
 template <typename Tin, typename Tout, typename T, int LOGN, bool ACCUM, int KIND, int TILE_>
 __global__ __launch_bounds__((TileCfg<LOGN, T, TILE_>::NT)) void xaxis_dst_kernel(
     const BatchPtr<const Tin> in, const BatchPtr<Tout> out, const long nrows, const T scale,
-    const T* __restrict__ tables, const int* __restrict__ done, int* __restrict__ reset) {
+    const T* __restrict__ tables, const int* __restrict__ done, int* __restrict__ reset,
+    const int tiles_pp, const int rows_pp) {
     using C = TileCfg<LOGN, T, TILE_>;
     using S = DstShape<LOGN>;
     using IO = PencilIO<KIND, LOGN>;
@@ -122,8 +124,13 @@ __global__ __launch_bounds__((TileCfg<LOGN, T, TILE_>::NT)) void xaxis_dst_kerne
     extern __shared__ __align__(16) unsigned char smem_raw[];
     T* lds = reinterpret_cast<T*>(smem_raw);
     const int tid = threadIdx.x;
-    const long r0 = (long)blockIdx.x * TILE;
-    const int rows_here = (int)((nrows - r0) < TILE ? (nrows - r0) : TILE);
+    long r0 = (long)blockIdx.x * TILE, left = nrows - r0;
+    if (tiles_pp > 0) {
+        const int pl = (int)blockIdx.x / tiles_pp, tr = ((int)blockIdx.x - pl * tiles_pp) * TILE;
+        r0 = (long)pl * rows_pp + tr;
+        left = rows_pp - tr;
+    }
+    const int rows_here = (int)(left < TILE ? left : TILE);
     // the tile's rows through buffer resources sized to the rows present:
     // rows past the last one read 0 and their stores are dropped
     const unsigned pts = (unsigned)rows_here * n;
@@ -303,11 +310,12 @@ static hipError_t xaxis_k(const AxisArgs& a) {
     const size_t lds = C::lds();
     hipError_t e = allow_lds(k, lds);
     if (e != hipSuccess) return e;
-    const long tiles = (a.nrows + C::TILE - 1) / C::TILE;
+    const int tpp = a.rows_per_plane > 0 ? (a.rows_per_plane + C::TILE - 1) / C::TILE : 0;
+    const long tiles = tpp ? a.nrows / a.rows_per_plane * tpp : (a.nrows + C::TILE - 1) / C::TILE;
     const BatchPtr<const Tin> in{(const Tin*)a.in, a.in_tab, a.bs_in};
     const BatchPtr<Tout> out{(Tout*)a.out, a.out_tab, a.bs_out};
     hipLaunchKernelGGL(k, dim3((unsigned)tiles, a.batch), dim3(C::NT), lds, a.stream, in, out, a.nrows,
-                       (T)a.scale, (const T*)a.tables, a.done, a.reset);
+                       (T)a.scale, (const T*)a.tables, a.done, a.reset, tpp, a.rows_per_plane);
     return hipGetLastError();
 }
 

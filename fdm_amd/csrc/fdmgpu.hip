@@ -295,6 +295,24 @@ bool variant_valid(const fdmgpu_plan_t* P, const Variant& v) {
 
 namespace {
 
+// FP32 transforms of 256 x 256 planes: the default variant (tile sizes 0) takes
+// the register kernel when a launch has this many planes, else the axis tiles
+// at their default sizes; both give the same bits.  A block of the register
+// kernel owns a plane and takes the same time whatever their number, the tiles
+// spread few planes over the GPU.  Measured (tiles / register kernel, us a
+// solve): 63 planes 76 / 85, 127 planes 89 / 93, 4 x 63 planes 150 / 122, 255
+// planes 153 / 117, 4 x 127 planes 276 / 223 in FP32; 63 planes 213 / 232, 255
+// planes 519 / 410, 4 x 63 planes 492 / 400 in FP32+refine.
+constexpr long kPlaneRegPlanes = 192;
+
+bool reg_shape(const fdmgpu_plan_t* P) {
+    return P->kind == 3 && P->precision != FDMGPU_F64 && P->logx == 8 && P->logy == 8;
+}
+bool use_plane_reg(const fdmgpu_plan_t* P, int count) {
+    return reg_shape(P) && !P->var.plane && !P->var.tile_x && !P->var.tile_y &&
+           (long)P->nz * count >= kPlaneRegPlanes;
+}
+
 // Records HIP events around one launch when timing is enabled.
 struct Timed {
     fdmgpu_plan_t* P;
@@ -381,10 +399,20 @@ int stage_fwd(fdmgpu_plan_t* P, const void* in, Tab in_tab, void* out, Tab out_t
         HIPCHK((launch_plane_rect<Tin, T, T>(P->logx, P->logy, a)));
         return FDMGPU_OK;
     }
+    if constexpr (std::is_same_v<T, float>) {
+        if (use_plane_reg(P, count)) {
+            PlaneArgs a{in, out, elems, elems, P->nz, count, sx, sy, P->tab_x, s, false, done, P->kfwd, in_tab, out_tab};
+            a.reset = reset;
+            Timed tm(P, plane_class, s);
+            HIPCHK((launch_plane_reg<Tin, float>(a)));
+            return FDMGPU_OK;
+        }
+    }
     if (P->kind == 3) {
         AxisArgs ax{in, out, (long)P->ny * P->nz, P->nx, P->nz, elems, elems, count, sx, P->tab_x, s, false, done,
                     P->kfwd, in_tab, out_tab, P->var.tile_x};
         ax.reset = reset;
+        if (reg_shape(P)) ax.rows_per_plane = P->ny;   // the register kernel's pencil pairs
         {
             Timed tm(P, FDMGPU_K_X_TILE, s);
             HIPCHK((launch_xaxis<Tin, T, T>(P->logx, ax)));
@@ -450,7 +478,17 @@ int stage_inv(fdmgpu_plan_t* P, void* in, Tab in_tab, void* out, Tab out_tab, in
         HIPCHK((launch_plane_rect<T, Tout, T>(P->logx, P->logy, a)));
         return FDMGPU_OK;
     }
-    if (base) return FDMGPU_ERR_INVALID_ARG;   // only the plane path adds onto a separate base
+    if constexpr (std::is_same_v<T, float>) {
+        if (use_plane_reg(P, count)) {
+            PlaneArgs a{in, out, elems, elems, P->nz, count, sx, sy, P->tab_x, s, accum, done, P->kinv, in_tab, out_tab,
+                        base};
+            a.inverse = true;
+            Timed tm(P, accum ? FDMGPU_K_XY_INV_ACC : FDMGPU_K_XY_INV, s);
+            HIPCHK((launch_plane_reg<float, Tout>(a)));
+            return FDMGPU_OK;
+        }
+    }
+    if (base) return FDMGPU_ERR_INVALID_ARG;   // only the plane kernels add onto a separate base
     if (P->kind == 3) {
         AxisArgs ay{in, in, 0, P->nx, P->nz, elems, elems, count, sy, P->tab_y, s, false, done, P->kinv, in_tab,
                     in_tab, P->var.tile_y};
@@ -460,6 +498,7 @@ int stage_inv(fdmgpu_plan_t* P, void* in, Tab in_tab, void* out, Tab out_tab, in
         }
         AxisArgs ax{in, out, (long)P->ny * P->nz, P->nx, P->nz, elems, elems, count, sx, P->tab_x, s, accum, done,
                     P->kinv, in_tab, out_tab, P->var.tile_x};
+        if (reg_shape(P)) ax.rows_per_plane = P->ny;
         Timed tm(P, FDMGPU_K_X_TILE, s);
         HIPCHK((launch_xaxis<T, Tout, T>(P->logx, ax)));
         return FDMGPU_OK;
@@ -694,8 +733,8 @@ int solve_refine(fdmgpu_plan_t* P, Work& W, double* ans, Tab ans_tab, const doub
     };
     // u1 in FP32 scratch: separate-residual plane path (Dirichlet planes), solves 1 and 2 in
     // this call (the fused forward pass reads an FP32 iterate slower than it saves)
-    const bool u1f = plane_capable(P) && P->var.plane && !fused && P->kinv == kDst && W.u32 && first == 1 &&
-                     last >= 2;
+    const bool u1f = ((plane_capable(P) && P->var.plane && !fused) || use_plane_reg(P, count)) && P->kinv == kDst &&
+                     W.u32 && first == 1 && last >= 2;
 
     // Fused path (cubes whose planes fit LDS): the forward DST of solve i >= 2
     // computes r = f - A u itself; convergence of the iterate after solve i is

@@ -116,6 +116,7 @@ struct PlaneArgs {
     bool stream_planes = false;   // plane_stream_kernel: FP64, N = 128, plain (no accum / base / done)
     const void* tables_y = nullptr;   // rectangular planes: the y axis's DST tables (tables: x)
     int* reset = nullptr;         // per batch item: set to 0 by the launch (one-plane-per-block kernels), or null
+    bool inverse = false;         // plane_reg_kernel: columns first, then rows
 };
 
 struct AxisArgs {
@@ -135,6 +136,7 @@ struct AxisArgs {
     const void* const* out_tab;
     int tile;             // pencils per block (16/32/64; 0 = default_tile)
     int* reset = nullptr; // per batch item: set to 0 by the launch, or null
+    int rows_per_plane = 0;   // x: > 0: tiles hold rows of one plane of so many rows (0: any consecutive rows)
 };
 
 struct ZcrArgs {
@@ -210,6 +212,9 @@ struct PlaneResidArgs {
 
 template <typename Tin, typename Tout, typename T>
 hipError_t launch_plane(int logn, const PlaneArgs& a);
+// FP32 planes of N = 256 (plane_reg_kernels.hip)
+template <typename Tin, typename Tout>
+hipError_t launch_plane_reg(const PlaneArgs& a);
 template <typename Tu>
 hipError_t launch_plane_resid(int logn, const PlaneResidArgs& a);
 template <typename T>
