@@ -482,18 +482,25 @@ __global__ __launch_bounds__(256) void zcrp_kernel(const BatchPtr<Ts> data, cons
 // LaplCyl3FFT2's r systems (src/lapl_cyl.cpp:55-73) are the same family with a
 // second eigenvalue: row k = i*rdiv + kz, D_j = -2/dr^2 - lm_phi[i]/r_j^2 -
 // lm_z[kz] (lmy = lm_phi, s_j = 1/r_j^2, lmz = lm_z).
-// One block per row; coefficients and rhs staged in LDS.
+// One block per row; coefficients and rhs staged in LDS.  Rows of up to 1024
+// points take rowpart_kernel below.
+// Instead of the diagonal a row carries its excess s_j = -D_j - L_j - U_j over the
+// couplings, exact at the start and updated by sums of positive terms (as
+// Grassmann, Taksar and Heyman's elimination does): the near-cancellation of
+// diagonal and couplings, where the lowest modes lose digits, never happens.
+// The arithmetic is FP64 also for FP32 data.
 // ---------------------------------------------------------------------------
-template <typename Ts, typename T>
+template <typename Ts>
 __global__ __launch_bounds__(256) void rowcr_kernel(const BatchPtr<Ts> data, const int nx, const int q,
                                                     const Ts* __restrict__ lmy, const Ts* __restrict__ sc,
                                                     const Ts* __restrict__ Ls, const Ts* __restrict__ Us,
                                                     const double inv_dx2, const int* __restrict__ done,
                                                     const Ts* __restrict__ lmz, const int rdiv) {
+    using T = double;
     if (done && done[blockIdx.y]) return;
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    T* d = reinterpret_cast<T*>(smem_raw);
-    T* e = d + nx;
+    T* s = reinterpret_cast<T*>(smem_raw);
+    T* e = s + nx;
     T* f = e + nx;
     T* bb = f + nx;
     const int k = blockIdx.x;
@@ -501,24 +508,27 @@ __global__ __launch_bounds__(256) void rowcr_kernel(const BatchPtr<Ts> data, con
     const Ts lk = lmy[lmz ? k / rdiv : k];
     const double lz = lmz ? (double)lmz[k % rdiv] : 0.0;
     for (int j = threadIdx.x; j < nx; j += blockDim.x) {
-        d[j] = lmz ? (T)(-2.0 * inv_dx2 - (double)(lk * sc[j]) - lz) : (T)(-2.0 * inv_dx2 - (double)(lk * sc[j]));
-        e[j] = j > 0 ? (T)(Ls[j] * inv_dx2) : T(0);
-        f[j] = j < nx - 1 ? (T)(Us[j] * inv_dx2) : T(0);
+        const T d = lmz ? -2.0 * inv_dx2 - (double)(lk * sc[j]) - lz : -2.0 * inv_dx2 - (double)(lk * sc[j]);
+        const T ej = j > 0 ? (T)(Ls[j] * inv_dx2) : T(0), fj = j < nx - 1 ? (T)(Us[j] * inv_dx2) : T(0);
+        e[j] = ej;
+        f[j] = fj;
+        s[j] = (-d - ej) - fj;
         bb[j] = (T)row[j];
     }
     __syncthreads();
+    auto diag = [&](const int j) { return e[j] + f[j] + s[j]; };
     for (int l = 1; l < q; ++l) {
         const int st = 1 << l, h = st >> 1;
         for (int j = st - 1 + threadIdx.x * st; j < nx; j += blockDim.x * st) {
-            const T alpha = -e[j] / d[j - h];
+            const T alpha = e[j] / diag(j - h);
             if (j + h < nx) {
-                const T gamma = -f[j] / d[j + h];
-                d[j] += alpha * f[j - h] + gamma * e[j + h];
+                const T gamma = f[j] / diag(j + h);
+                s[j] += alpha * s[j - h] + gamma * s[j + h];
                 bb[j] += alpha * bb[j - h] + gamma * bb[j + h];
                 e[j] = alpha * e[j - h];
                 f[j] = gamma * f[j + h];
             } else {
-                d[j] += alpha * f[j - h];
+                s[j] += alpha * s[j - h];
                 bb[j] += alpha * bb[j - h];
                 e[j] = alpha * e[j - h];
             }
@@ -526,22 +536,177 @@ __global__ __launch_bounds__(256) void rowcr_kernel(const BatchPtr<Ts> data, con
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        int top = (1 << (q - 1)) - 1;
-        if (top > nx - 1) top = nx - 1;
-        bb[top] = bb[top] / d[top];
+        const int top = (1 << (q - 1)) - 1;   // <= nx - 1
+        bb[top] = -bb[top] / diag(top);
     }
     __syncthreads();
     for (int l = q - 1; l > 0; --l) {
         const int st = 1 << l, h = st >> 1;
         for (int j = h - 1 + threadIdx.x * st; j < nx; j += blockDim.x * st) {
-            T acc = bb[j];
-            if (j - h >= 0) acc -= e[j] * bb[j - h];
-            if (j + h < nx) acc -= f[j] * bb[j + h];
-            bb[j] = acc / d[j];
+            T acc = -bb[j];
+            if (j - h >= 0) acc += e[j] * bb[j - h];
+            if (j + h < nx) acc += f[j] * bb[j + h];
+            bb[j] = acc / diag(j);
         }
         __syncthreads();
     }
     for (int j = threadIdx.x; j < nx; j += blockDim.x) row[j] = (Ts)bb[j];
+}
+
+// ---------------------------------------------------------------------------
+// The same row systems (nx <= 1024) with one wavefront per row and everything in
+// registers: lane t owns C consecutive unknowns, the last of them a separator.
+// Its C - 1 interior unknowns are eliminated (Thomas on the right-hand side and
+// the two coupling columns together), which leaves x_i = b_i + l_i xL + r_i xS in
+// terms of the separators left of and in the chunk; the separators' tridiagonal
+// system over the lanes is solved by parallel cyclic reduction (lanes' values by
+// shuffles), and the chunk follows from its two separators.
+// Rows carry their excess s = -d - a - c as in rowcr_kernel.  Error against extended precision, rows of 511 / 1000 points, lowest mode:
+// cyclic reduction 8e-13 / 3e-12, this 1e-15 / 2e-15.  No barrier, and C +
+// log2 of the lanes dependent reciprocals where rowcr_kernel's 2 log2(nx) levels
+// each wait for LDS, a division and a barrier: 511 FP64 rows of 511 points 11.3
+// us there, 5.2 here.  The row is read and written coalesced and turned
+// through LDS (chunk stride C + 1: conflict-free).
+// The arithmetic is FP64 also for FP32 data: the lowest modes' systems are nearly
+// singular (in FP32 the refinement of 511 x 1000 points with a smooth right-hand
+// side stopped at 1.3e-10 after four inner solves).
+// UNIFORM: unit scales, so the coefficients are 1/dx^2 and one diagonal a row.
+// ---------------------------------------------------------------------------
+constexpr int kRowWaves = 2;   // rows per block: many small blocks for the few rows of one problem
+
+template <typename Ts, int C, bool UNIFORM>
+__global__ __launch_bounds__(64 * kRowWaves) void rowpart_kernel(
+    const BatchPtr<Ts> data, const int nx, const int nrows, const Ts* __restrict__ lmy, const Ts* __restrict__ sc,
+    const Ts* __restrict__ Ls, const Ts* __restrict__ Us, const double inv_dx2, const int* __restrict__ done,
+    const Ts* __restrict__ lmz, const int rdiv) {
+    using T = double;
+    if (done && done[blockIdx.y]) return;
+    constexpr int M = C - 1;   // interior unknowns of a lane
+    __shared__ Ts turn[kRowWaves][C > 1 ? 64 * (C + 1) : 1];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int k = (int)blockIdx.x * kRowWaves + wv;
+    if (k >= nrows) return;   // whole waves; no block barrier below
+    const auto row = as_global(data(blockIdx.y) + (long)k * nx);
+    Ts raw[C];
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+        const int j = 64 * i + lane;
+        raw[i] = row[j < nx ? j : nx - 1];
+    }
+    const Ts lk = lmy[lmz ? k / rdiv : k];
+    const double lz = lmz ? (double)lmz[k % rdiv] : 0.0;
+    Ts* const sh = turn[wv];
+    auto pos = [](const int j) { return j / C * (C + 1) + j % C; };   // chunk-major, stride C + 1
+    T b[C];
+    if constexpr (C > 1) {
+#pragma unroll
+        for (int i = 0; i < C; ++i) sh[pos(64 * i + lane)] = raw[i];
+        wave_lds_sync();
+#pragma unroll
+        for (int i = 0; i < C; ++i) b[i] = (T)sh[lane * (C + 1) + i];
+        wave_lds_sync();
+    } else {
+        b[0] = (T)raw[0];
+    }
+    // row j: a x_(j-1) - (a + c + s) x_j + c x_(j+1) = b; rows past nx are x = 0
+    T a[C], s[C], c[C];
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+        const int j = lane * C + i;
+        const bool in = j < nx;
+        T dv, av, cv;
+        if constexpr (UNIFORM) {
+            dv = (T)(-2.0 * inv_dx2 - (double)lk);
+            av = cv = (T)inv_dx2;
+        } else {
+            const int jc = in ? j : nx - 1;
+            dv = lmz ? (T)(-2.0 * inv_dx2 - (double)(lk * sc[jc]) - lz) : (T)(-2.0 * inv_dx2 - (double)(lk * sc[jc]));
+            av = (T)(Ls[jc] * inv_dx2);
+            cv = (T)(Us[jc] * inv_dx2);
+        }
+        a[i] = in && j > 0 ? av : T(0);
+        c[i] = j < nx - 1 ? cv : T(0);
+        s[i] = in ? (-dv - a[i]) - c[i] : T(1);
+        if (!in) b[i] = T(0);
+    }
+    // interior: x_i = b_i + l_i xL + r_i xS, with s_i = 1 - l_i - r_i
+    T l[C], r[C];
+    if constexpr (M > 0) {
+        T inv[C];
+        l[0] = a[0];
+        inv[0] = T(1) / (l[0] + s[0] + c[0]);
+#pragma unroll
+        for (int i = 1; i < M; ++i) {
+            const T w = a[i] * inv[i - 1];
+            b[i] += w * b[i - 1];
+            l[i] = w * l[i - 1];
+            s[i] += w * s[i - 1];
+            inv[i] = T(1) / (l[i] + s[i] + c[i]);
+        }
+        b[M - 1] *= -inv[M - 1];
+        l[M - 1] *= inv[M - 1];
+        s[M - 1] *= inv[M - 1];
+        r[M - 1] = c[M - 1] * inv[M - 1];
+#pragma unroll
+        for (int i = M - 2; i >= 0; --i) {
+            const T t = c[i] * inv[i];
+            b[i] = t * b[i + 1] - b[i] * inv[i];
+            l[i] = l[i] * inv[i] + t * l[i + 1];
+            s[i] = s[i] * inv[i] + t * s[i + 1];
+            r[i] = t * r[i + 1];
+        }
+    }
+    // separators: x = A xL + G xR + B, S = 1 - A - G
+    T A = a[M], S = s[M], G = c[M], B = b[M];
+    if constexpr (M > 0) {
+        const T bn = __shfl_down(b[0], 1, 64), sn = __shfl_down(s[0], 1, 64), rn = __shfl_down(r[0], 1, 64);
+        S += a[M] * s[M - 1] + c[M] * sn;
+        B -= a[M] * b[M - 1] + c[M] * bn;
+        A = a[M] * l[M - 1];
+        G = c[M] * rn;
+    }
+    {
+        const T iv = T(1) / (A + G + S);
+        A *= iv;
+        G *= iv;
+        S *= iv;
+        B *= -iv;
+    }
+    // (A is 0 where the left neighbour does not exist, G where the right one does
+    // not: what a shuffle past the end returns is multiplied by it)
+    const int lanes = (nx + C - 1) / C;
+    for (int h = 1; h < lanes; h <<= 1) {
+        const T Al = __shfl_up(A, h, 64), Sl = __shfl_up(S, h, 64), Bl = __shfl_up(B, h, 64);
+        const T Gr = __shfl_down(G, h, 64), Sr = __shfl_down(S, h, 64), Br = __shfl_down(B, h, 64);
+        S += A * Sl + G * Sr;
+        B += A * Bl + G * Br;
+        A *= Al;
+        G *= Gr;
+        const T iv = T(1) / (A + G + S);
+        A *= iv;
+        G *= iv;
+        S *= iv;
+        B *= iv;
+    }
+    if constexpr (M > 0) {
+        T xL = __shfl_up(B, 1, 64);
+        if (lane == 0) xL = T(0);
+#pragma unroll
+        for (int i = 0; i < M; ++i) b[i] += l[i] * xL + r[i] * B;
+        b[M] = B;
+#pragma unroll
+        for (int i = 0; i < C; ++i) sh[lane * (C + 1) + i] = (Ts)b[i];
+        wave_lds_sync();
+#pragma unroll
+        for (int i = 0; i < C; ++i) raw[i] = sh[pos(64 * i + lane)];
+    } else {
+        raw[0] = (Ts)B;
+    }
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+        const int j = 64 * i + lane;
+        if (j < nx) row[j] = raw[i];
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -702,15 +867,31 @@ hipError_t launch_zcr(int q, const ZcrArgs& a) {
     }
 }
 
-template <typename Ts, typename T>
+template <typename Ts, int C>
+static hipError_t rowpart_k(const RowCrArgs& a) {
+    auto k = a.uniform ? rowpart_kernel<Ts, C, true> : rowpart_kernel<Ts, C, false>;
+    const BatchPtr<Ts> data{(Ts*)a.data, a.data_tab, a.bs};
+    hipLaunchKernelGGL(k, dim3((a.nrows + kRowWaves - 1) / kRowWaves, a.batch), dim3(64 * kRowWaves), 0, a.stream,
+                       data, a.nx, a.nrows, (const Ts*)a.lmy, (const Ts*)a.sc, (const Ts*)a.Ls, (const Ts*)a.Us,
+                       a.inv_dx2, a.done, (const Ts*)a.lmz, a.rdiv);
+    return hipGetLastError();
+}
+
+template <typename Ts>
 static hipError_t rowcr_k(const RowCrArgs& a) {
+    // the fewest unknowns a lane that cover the row; longer rows by LDS
+    if (a.nx <= 64) return rowpart_k<Ts, 1>(a);
+    if (a.nx <= 128) return rowpart_k<Ts, 2>(a);
+    if (a.nx <= 256) return rowpart_k<Ts, 4>(a);
+    if (a.nx <= 512) return rowpart_k<Ts, 8>(a);
+    if (a.nx <= 1024) return rowpart_k<Ts, 16>(a);
     int q = 0;
     while ((1 << q) < a.nx + 1) q++;
-    const size_t lds = 4 * sizeof(T) * (size_t)a.nx;
-    hipError_t e = allow_lds(rowcr_kernel<Ts, T>, lds);
+    const size_t lds = 4 * sizeof(double) * (size_t)a.nx;
+    hipError_t e = allow_lds(rowcr_kernel<Ts>, lds);
     if (e != hipSuccess) return e;
     const BatchPtr<Ts> data{(Ts*)a.data, a.data_tab, a.bs};
-    hipLaunchKernelGGL((rowcr_kernel<Ts, T>), dim3(a.nrows, a.batch), dim3(256), lds, a.stream, data, a.nx, q,
+    hipLaunchKernelGGL((rowcr_kernel<Ts>), dim3(a.nrows, a.batch), dim3(256), lds, a.stream, data, a.nx, q,
                        (const Ts*)a.lmy, (const Ts*)a.sc, (const Ts*)a.Ls, (const Ts*)a.Us, a.inv_dx2, a.done,
                        (const Ts*)a.lmz, a.rdiv);
     return hipGetLastError();
@@ -718,7 +899,7 @@ static hipError_t rowcr_k(const RowCrArgs& a) {
 
 template <typename Ts, typename T>
 static hipError_t rowgtsv_k(const RowCrArgs& a) {
-    const size_t lds = 4 * sizeof(T) * (size_t)a.nx;
+    const size_t lds = 4 * sizeof(double) * (size_t)a.nx;
     hipError_t e = allow_lds(rowgtsv_kernel<Ts, T>, lds);
     if (e != hipSuccess) return e;
     const BatchPtr<Ts> data{(Ts*)a.data, a.data_tab, a.bs};
@@ -736,10 +917,7 @@ hipError_t launch_rowcr(const RowCrArgs& a) {
         }
         return rowgtsv_k<T, T>(a);
     }
-    if constexpr (std::is_same_v<T, float>) {
-        if (a.wide) return rowcr_k<float, double>(a);
-    }
-    return rowcr_k<T, T>(a);
+    return rowcr_k<T>(a);
 }
 
 // ---------------------------------------------------------------------------

@@ -305,6 +305,12 @@ namespace {
 // planes 519 / 410, 4 x 63 planes 492 / 400 in FP32+refine.
 constexpr long kPlaneRegPlanes = 192;
 
+// Columns per block of a 2-D plan's y transforms by default: 16, so that the few
+// columns of one problem reach more CUs (one solve in FP64, tiles of 32 / 16 / 64
+// columns, us: 511 x 511 40 / 33 / -, 255 x 255 23 / 20 / 33, 127 x 127 18 / 17 /
+// 22; 50 problems a solve: 192 / 195, 53 / 55, 30 / 30).
+int rect_tile_y(const fdmgpu_plan_t* P) { return P->var.tile_y ? P->var.tile_y : 16; }
+
 bool reg_shape(const fdmgpu_plan_t* P) {
     return P->kind == 3 && P->precision != FDMGPU_F64 && P->logx == 8 && P->logy == 8;
 }
@@ -425,7 +431,7 @@ int stage_fwd(fdmgpu_plan_t* P, const void* in, Tab in_tab, void* out, Tab out_t
     }
     // rect: y (LaplRectFFT2: then x)
     AxisArgs ay{in, out, 0, P->nx, 1, elems, elems, count, sy, P->tab_y, s, false, done, P->kfwd, in_tab, out_tab,
-                P->var.tile_y};
+                rect_tile_y(P)};
     ay.reset = reset;
     {
         Timed tm(P, FDMGPU_K_Y_TILE, s);
@@ -511,13 +517,13 @@ int stage_inv(fdmgpu_plan_t* P, void* in, Tab in_tab, void* out, Tab out_tab, in
     }
     if (accum) {   // rect: inverse y into the FP32 buffer, then accumulate through an x pass-free add
         AxisArgs ay{in, in, 0, P->nx, 1, elems, elems, count, sy, P->tab_y, s, false, done, P->kinv, in_tab, in_tab,
-                    P->var.tile_y};
+                    rect_tile_y(P)};
         Timed tm(P, FDMGPU_K_Y_TILE, s);
         HIPCHK((launch_yaxis<T, T, T>(P->logy, ay)));
         return -1;   // caller adds
     }
     AxisArgs ay{in, out, 0, P->nx, 1, elems, elems, count, sy, P->tab_y, s, false, done, P->kinv, in_tab, out_tab,
-                P->var.tile_y};
+                rect_tile_y(P)};
     Timed tm(P, FDMGPU_K_Y_TILE, s);
     HIPCHK((launch_yaxis<T, Tout, T>(P->logy, ay)));
     return FDMGPU_OK;
@@ -558,6 +564,7 @@ int stage_tridiag(fdmgpu_plan_t* P, void* data, Tab data_tab, int count, hipStre
     RowCrArgs r{data, P->nx, P->ny, P->lmy, P->d_sc, P->d_Ls, P->d_Us, 1.0 / (P->dx * P->dx), elems, count, s, done,
                 P->precision == FDMGPU_F32, data_tab};
     r.pivot = P->pivot_rows;
+    r.uniform = !P->scaled;
     Timed tm(P, FDMGPU_K_ROWCR, s);
     HIPCHK(launch_rowcr<T>(r));
     return FDMGPU_OK;

@@ -172,6 +172,7 @@ struct RowCrArgs {
     const void* const* data_tab;
     const void* lmz = nullptr;   // LaplCyl3FFT2: second per-row eigenvalue, row k uses lmy[k / rdiv] and
     int rdiv = 1;                //   lmz[k % rdiv] (D_j = -2/dx^2 - lmy*s_j - lmz)
+    bool uniform = false;        // unit scales (sc, Ls, Us all 1) and no lmz
     bool pivot = false;          // Gaussian elimination with partial pivoting (rows that are not
                                  //   diagonally dominant) instead of cyclic reduction
 };
