@@ -1267,10 +1267,18 @@ int fdmgpu_solve_host(fdmgpu_plan plan, void* ans, const void* rhs) {
     if (!plan->own) HIPCHK(hipStreamCreateWithFlags(&plan->own, hipStreamNonBlocking));
     char* d_rhs = (char*)plan->stage;
     char* d_ans = plan->precision == FDMGPU_F32_REFINE64 ? d_rhs + bytes : d_rhs;
-    HIPCHK(hipMemcpyAsync(d_rhs, rhs, bytes, hipMemcpyHostToDevice, plan->own));
+    // a plan that solves once does not pay for setting a stage up
+    if (!plan->host_st && bytes >= kStageMin) plan->host_st = host_stage(plan->device, plan->host_calls > 0);
+    if (plan->host_calls < 2) plan->host_calls++;
+    HostStage* const st = bytes >= kStageMin ? plan->host_st.get() : nullptr;
+    hipError_t e = st ? stage_in(*st, d_rhs, rhs, bytes, plan->own) : hipErrorNotReady;
+    if (e == hipErrorNotReady) e = hipMemcpyAsync(d_rhs, rhs, bytes, hipMemcpyHostToDevice, plan->own);
+    HIPCHK(e);
     int rc = solve_device_impl(plan, d_ans, nullptr, d_rhs, nullptr, 1, plan->own);
     if (rc) return rc;
-    HIPCHK(hipMemcpyAsync(ans, d_ans, bytes, hipMemcpyDeviceToHost, plan->own));
+    e = st ? stage_out(*st, ans, d_ans, bytes, plan->own) : hipErrorNotReady;
+    if (e == hipErrorNotReady) e = hipMemcpyAsync(ans, d_ans, bytes, hipMemcpyDeviceToHost, plan->own);
+    HIPCHK(e);
     HIPCHK(hipStreamSynchronize(plan->own));
     if (plan->precision == FDMGPU_F32_REFINE64) {
         fdmgpu_stats st;

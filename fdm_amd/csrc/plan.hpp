@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "../../include/fdmgpu.h"
+#include "host_stage.hpp"
 
 namespace fdmgpu {
 
@@ -85,6 +86,8 @@ struct fdmgpu_plan_t {
     void* stage = nullptr;
     size_t stage_bytes = 0;
     hipStream_t own = nullptr;
+    std::shared_ptr<fdmgpu::HostStage> host_st;   // held from the plan's second host solve on (or
+    int host_calls = 0;                           //   the first, if another plan holds it)
     hipStream_t last_stream = nullptr;
     int last_count = 0;
     const int* last_iters = nullptr;    // per-problem results of the last refine solve (device):
