@@ -131,7 +131,7 @@ __device__ __forceinline__ void cr_dirichlet_lanes(T (&v)[(ZcrCfg<T, Q, GM>::C)]
 template <typename Ts, typename T, int Q, int GM>
 __global__ __launch_bounds__(256) void zcr_kernel(const BatchPtr<Ts> data, const long plane, const int nx,
                                                   const Ts* __restrict__ lmx, const Ts* __restrict__ lmy,
-                                                  const T b, const T d0, const T gamma,
+                                                  const T b, const T gamma,
                                                   const int* __restrict__ done, const long blocks,
                                                   const int batch) {
     using Cf = ZcrCfg<T, Q, GM>;
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256) void zcr_kernel(const BatchPtr<Ts> data, const
         v[r] = (valid && row < NQ - 1) ? x * gamma : T(0);
     }
     CrLevels<T, Q> L;
-    cr_levels<T, Q>(L, b, d0 - (T)lmx[kx] - (T)lmy[ky]);
+    cr_levels<T, Q>(L, b, (T)lmx[kx] + (T)lmy[ky]);
     cr_dirichlet_lanes<T, Q, GM>(v, L, lane, s, c);
 
     if (valid) {
@@ -194,7 +194,7 @@ struct ZcrStripCfg {
 template <typename Ts, typename T, int Q, int S, int CR>
 __global__ __launch_bounds__((64 * ZcrStripCfg<Q, CR>::G * S)) void zcr_strip_kernel(
     const BatchPtr<Ts> data, const long plane, const int nx, const Ts* __restrict__ lmx,
-    const Ts* __restrict__ lmy, const T b, const T d0, const T gamma, const int* __restrict__ done,
+    const Ts* __restrict__ lmy, const T b, const T gamma, const int* __restrict__ done,
     const int blocks, const int batch) {
     using Cf = ZcrStripCfg<Q, CR>;
     constexpr int NQ = Cf::NQ, C = Cf::C, G = Cf::G, LOGG = Cf::LOGG, LOC = Cf::LOC;
@@ -222,7 +222,7 @@ __global__ __launch_bounds__((64 * ZcrStripCfg<Q, CR>::G * S)) void zcr_strip_ke
         v[r] = (valid && row < NQ - 1) ? x * gamma : T(0);
     }
     CrLevels<T, Q> L;
-    cr_levels<T, Q>(L, b, d0 - (T)lmx[kx] - (T)lmy[ky]);
+    cr_levels<T, Q>(L, b, (T)lmx[kx] + (T)lmy[ky]);
 
     // forward reduction inside the chunk
     T toRight = T(0), toLeft = T(0);
@@ -329,18 +329,13 @@ struct CrLevelsP {
 };
 
 template <typename T, int Q>
-__device__ __forceinline__ void cr_levels_periodic(CrLevelsP<T, Q>& L, T b, T d) {
-    T cl = b, dl = d;
+__device__ __forceinline__ void cr_levels_periodic(CrLevelsP<T, Q>& L, T c, T s) {
 #pragma unroll
     for (int l = 0; l < Q; ++l) {
-        L.c[l] = cl;
-        L.inv_d[l] = T(1) / dl;
-        const T t = cl * cl * L.inv_d[l];
-        L.alpha[l + 1] = -cl * L.inv_d[l];
-        dl = dl - T(2) * t;
-        cl = -t;
+        L.c[l] = c;
+        cr_level(c, s, L.inv_d[l], L.alpha[l + 1]);
     }
-    L.inv_top = T(1) / (dl + T(2) * cl);
+    L.inv_top = T(-1) / s;   // d_Q + 2 c_Q = -s_Q
 }
 
 // sum of x over the G lanes of one system (lanes s + i*W)
@@ -354,7 +349,7 @@ __device__ __forceinline__ T system_sum(T x) {
 template <typename Ts, typename T, int Q, int GM>
 __global__ __launch_bounds__(256) void zcrp_kernel(const BatchPtr<Ts> data, const long plane, const int nx,
                                                    const Ts* __restrict__ lmx, const Ts* __restrict__ lmy,
-                                                   const T b, const T d0, const T gamma,
+                                                   const T b, const T gamma,
                                                    const int* __restrict__ done, const long blocks,
                                                    const int batch) {
     using Cf = ZcrCfg<T, Q, GM>;
@@ -381,7 +376,7 @@ __global__ __launch_bounds__(256) void zcrp_kernel(const BatchPtr<Ts> data, cons
 
     if (mm != 0) {
         CrLevelsP<T, Q> L;
-        cr_levels_periodic<T, Q>(L, b, d0 - (T)lmx[kx] - (T)lmy[ky]);
+        cr_levels_periodic<T, Q>(L, b, (T)lmx[kx] + (T)lmy[ky]);
         T own = T(0), toNext = T(0);
         static_for<1, LOC + 1>([&](auto ll) {
             constexpr int l = decltype(ll)::value;
@@ -453,7 +448,7 @@ __global__ __launch_bounds__(256) void zcrp_kernel(const BatchPtr<Ts> data, cons
         for (int r = 0; r + 1 < C; ++r) v[r] = v[r + 1] - mean;
         v[C - 1] = nxt - mean;
         CrLevels<T, Q> Ld;
-        cr_levels<T, Q>(Ld, b, d0);
+        cr_levels<T, Q>(Ld, b, T(0));
         cr_dirichlet_lanes<T, Q, GM>(v, Ld, lane, s, c);
         T prev = T(0);
         if constexpr (G > 1) prev = __shfl(v[C - 1], (lane - W) & 63, 64);   // row c*C
@@ -800,7 +795,7 @@ static hipError_t zcr_k(const ZcrArgs& a) {
     auto k = a.periodic ? zcrp_kernel<Ts, T, Q, GM> : zcr_kernel<Ts, T, Q, GM>;
     const BatchPtr<Ts> data{(Ts*)a.data, a.data_tab, a.bs};
     hipLaunchKernelGGL(k, dim3(xcd_slab_grid(blocks, a.batch)), dim3(C::NT), 0, a.stream, data, a.plane, a.nx,
-                       (const Ts*)a.lmx, (const Ts*)a.lmy, (T)a.b, (T)a.d0, (T)a.gamma, a.done, blocks, a.batch);
+                       (const Ts*)a.lmx, (const Ts*)a.lmy, (T)a.b, (T)a.gamma, a.done, blocks, a.batch);
     return hipGetLastError();
 }
 
@@ -811,7 +806,7 @@ static hipError_t zcr_strip_k(const ZcrArgs& a) {
     const BatchPtr<Ts> data{(Ts*)a.data, a.data_tab, a.bs};
     hipLaunchKernelGGL((zcr_strip_kernel<Ts, T, Q, S, CR>), dim3(xcd_slab_grid(blocks, a.batch)),
                        dim3(64 * ZcrStripCfg<Q, CR>::G * S), 0, a.stream, data, a.plane, a.nx, (const Ts*)a.lmx,
-                       (const Ts*)a.lmy, (T)a.b, (T)a.d0, (T)a.gamma, a.done, blocks, a.batch);
+                       (const Ts*)a.lmy, (T)a.b, (T)a.gamma, a.done, blocks, a.batch);
     return hipGetLastError();
 }
 

@@ -787,6 +787,11 @@ __device__ __forceinline__ void dst_pairs128(T* __restrict__ lds, const Lane& L,
 // when n = 2^Q - 1, so each level is two scalars per mode:
 //   alpha_l = -c_{l-1}/d_{l-1},  d_l = d_{l-1} - 2 c_{l-1}^2/d_{l-1},
 //   c_l = -c_{l-1}^2/d_{l-1}.
+// The diagonal is carried as its excess s = -d - 2 c over the couplings (s_0 =
+// lambda_x + lambda_y), which a level multiplies by 1 + 2 alpha: every quantity
+// is a sum or product of positive terms, so the lowest modes' systems, where d
+// and 2 c nearly cancel, keep full relative accuracy.  (Carried as d, FP32
+// elimination loses 1e-4 of those modes at 128 rows, FP64 1e-13.)
 // G lanes share one system: lane c owns the contiguous chunk of rows
 // [c*C, (c+1)*C - 1) plus the separator row (c+1)*C - 1 (C = 2^Q/G).  The
 // lowest Q-g levels stay inside a chunk; the separators' updates are additive
@@ -801,19 +806,25 @@ struct CrLevels {
     T inv_d[Q];               // 1/d[l], l = 0..Q-1
 };
 
+// One level's scalars from (c, s), and the next level's (c, s).
+template <typename T>
+__device__ __forceinline__ void cr_level(T& c, T& s, T& inv_d, T& alpha) {
+    const T inv = T(1) / fma(T(2), c, s);   // -1/d
+    inv_d = -inv;
+    alpha = c * inv;
+    c *= alpha;
+    s = fma(T(2) * alpha, s, s);
+}
+
+// c = b, s = lambda_x + lambda_y
 template <typename T, int Q>
-__device__ __forceinline__ void cr_levels(CrLevels<T, Q>& L, T b, T d) {
-    T cl = b, dl = d;
-    L.c[0] = cl;
-    L.inv_d[0] = T(1) / dl;
+__device__ __forceinline__ void cr_levels(CrLevels<T, Q>& L, T c, T s) {
 #pragma unroll
-    for (int l = 1; l < Q; ++l) {
-        const T t = cl * cl * L.inv_d[l - 1];
-        L.alpha[l] = -cl * L.inv_d[l - 1];
-        dl = dl - T(2) * t;
-        cl = -t;
-        L.c[l] = cl;
-        L.inv_d[l] = T(1) / dl;
+    for (int l = 0; l < Q; ++l) {
+        L.c[l] = c;
+        T a;
+        cr_level(c, s, L.inv_d[l], a);
+        if (l + 1 < Q) L.alpha[l + 1] = a;
     }
 }
 

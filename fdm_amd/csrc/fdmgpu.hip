@@ -540,7 +540,7 @@ int stage_tridiag(fdmgpu_plan_t* P, void* data, Tab data_tab, int count, hipStre
     if (P->kind == 3) {
         const double b = 1.0 / (P->hz_op * P->hz_op);
         const double gamma = P->dz * (double)(1 << P->logz) / P->lz;
-        ZcrArgs z{data, (long)P->nx * P->ny, P->nx, P->lmx, P->lmy, b, -2.0 * b,
+        ZcrArgs z{data, (long)P->nx * P->ny, P->nx, P->lmx, P->lmy, b,
                   std::fabs(gamma - 1.0) < 4e-16 ? 1.0 : gamma, elems, count, s, done, P->periodic != 0,
                   P->precision == FDMGPU_F32, data_tab, P->var.zcr_gmul};
         Timed tm(P, FDMGPU_K_ZCR, s);

@@ -145,7 +145,7 @@ struct ZcrArgs {
     int nx;
     const void* lmx;      // eigenvalues per mode index (compute type)
     const void* lmy;
-    double b, d0, gamma;  // 1/hz^2, -2/hz^2, rhs scale
+    double b, gamma;      // 1/hz^2, rhs scale
     long bs;
     int batch;
     hipStream_t stream;
