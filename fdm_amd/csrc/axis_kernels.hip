@@ -279,6 +279,80 @@ __global__ __launch_bounds__((TileCfg<LOGN, T, TILE_>::NT)) void yaxis_dst_kerne
 }
 
 
+// Columns of planes with 255 or 511 rows (DST-I), a half or a whole wavefront to
+// each pair of columns (WaveDst).  Where few tiles are in flight the pass is a
+// chain of latencies, and eight points a lane make it half as long: a 2-D solve
+// of 511 x 511 points took 33.5 us and takes 19.9 (FP32 34.2 -> 17.6), 511 x 255
+// 21.3 -> 16.4; with the chip full the columns of 511 gain by holding 16
+// wavefronts a CU instead of 4 (64 x 511 x 511 FP64 215 -> 170 us, 255 x 511 x 63
+// 171 -> 152), those of 255 run at the rate of memory either way.
+// A pair is columns 2c and 2c + 1 of the plane whatever TILE is, so both tile
+// widths give the same bits.  The pitch spreads the copies between rows and
+// pencils over the banks.
+template <typename T, int LOGN, int TILE_>
+struct WaveTileCfg {
+    static constexpr int TILE = TILE_, NT = TILE / 2 * WaveDst<T, LOGN>::L;
+    static constexpr int P = (1 << LOGN) + (TILE == 8 ? 4 : sizeof(T) == 8 ? 17 : 2);
+    static constexpr size_t lds() { return sizeof(T) * (size_t)TILE * P; }
+};
+
+template <typename Tin, typename Tout, typename T, int LOGN, int TILE_>
+__global__ __launch_bounds__((WaveTileCfg<T, LOGN, TILE_>::NT)) __attribute__((amdgpu_waves_per_eu(TILE_ == 8 ? 2 : 4)))
+void yaxis_wave_kernel(
+    const BatchPtr<const Tin> in, const BatchPtr<Tout> out, const int nx, const T scale,
+    const T* __restrict__ tables, const int* __restrict__ done, const int nplanes, const int batch,
+    int* __restrict__ reset) {
+    using C = WaveTileCfg<T, LOGN, TILE_>;
+    using W = WaveDst<T, LOGN>;
+    constexpr int n = W::N - 1, NT = C::NT, TILE = C::TILE;
+    const int ntx = (nx + TILE - 1) / TILE;
+    const long per = (long)gridDim.x / kAxisXcds;
+    const long tile_id = ((long)blockIdx.x % kAxisXcds) * per + (long)blockIdx.x / kAxisXcds;
+    if (tile_id >= (long)ntx * nplanes * batch) return;
+    const int bx = (int)(tile_id % ntx);
+    const long rest = tile_id / ntx;
+    const int by = (int)(rest % nplanes), bz = (int)(rest / nplanes);
+    if (done && done[bz]) return;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    T* lds = reinterpret_cast<T*>(smem_raw);
+    const int tid = threadIdx.x;
+    const int x0 = bx * TILE;
+    const long poff = (long)by * n * nx;
+    // thread tid owns tile column p = tid % TILE and rows y0 + YR*i, y0 = tid / TILE
+    constexpr int YR = NT / TILE, YI = (n + YR - 1) / YR;
+    const unsigned pts = (unsigned)n * nx;
+    const BufRange<Tin> src(in(bz) + poff, pts * sizeof(Tin));
+    const BufRange<Tout> dst(out(bz) + poff, pts * sizeof(Tout));
+    const int p = tid % TILE, y0 = tid / TILE;
+    const bool col_ok = x0 + p < nx;
+    const int lane_in = (y0 * nx + (col_ok ? x0 + p : 0)) * (int)sizeof(Tin);
+    const int lane_out = (y0 * nx + (col_ok ? x0 + p : 0)) * (int)sizeof(Tout);
+    T* const pb = lds + p * C::P;
+    Tin v[YI] = {};
+#pragma unroll
+    for (int i = 0; i < YI; ++i)
+        if (YR * i + YR <= n || y0 + YR * i < n) v[i] = src.load(lane_in, YR * i * nx * (int)sizeof(Tin));
+    __builtin_amdgcn_sched_barrier(0);
+    W w;
+    w.init(tables, tid % W::L);
+    if (tid < TILE) lds[tid * C::P] = T(0);   // slot 0 of every pencil
+#pragma unroll
+    for (int i = 0; i < YI; ++i)
+        if (YR * i + YR <= n || y0 + YR * i < n) pb[y0 + YR * i + 1] = col_ok ? (T)v[i] : T(0);
+    __syncthreads();
+    T* const a = lds + tid / W::L * 2 * C::P;
+    w.pair(a, a + C::P, scale, tid % W::L);
+    __syncthreads();
+    if (col_ok) {
+#pragma unroll
+        for (int i = 0; i < YI; ++i) {
+            const int y = y0 + YR * i;
+            if (YR * i + YR <= n || y < n) dst.store((Tout)pb[W::out(y)], lane_out, YR * i * nx * (int)sizeof(Tout));
+        }
+    }
+    if (reset && bx == 0 && by == 0 && tid == 0) reset[bz] = 0;
+}
+
 // Tile sizes an axis kernel of length 2^logn supports: 16 always; 32 and 64
 // for N >= 32 when the tile (TILE x (N + N1) elements) fits LDS.
 template <typename T>
@@ -367,8 +441,35 @@ static hipError_t yaxis_k(const AxisArgs& a) {
 }
 
 template <typename Tin, typename Tout, typename T, int LOGN, int TILE>
+static hipError_t yaxis_wave_k(const AxisArgs& a) {
+    using C = WaveTileCfg<T, LOGN, TILE>;
+    auto k = yaxis_wave_kernel<Tin, Tout, T, LOGN, TILE>;
+    constexpr size_t elem = sizeof(Tin) > sizeof(Tout) ? sizeof(Tin) : sizeof(Tout);
+    if (((size_t)1 << LOGN) * (size_t)a.nx * elem >= ((size_t)1 << 31)) return hipErrorInvalidValue;
+    const hipError_t e = allow_lds(k, C::lds());
+    if (e != hipSuccess) return e;
+    const long tiles = (long)((a.nx + TILE - 1) / TILE) * a.nplanes * a.batch;
+    const long blocks = (tiles + kAxisXcds - 1) / kAxisXcds * kAxisXcds;
+    if (tiles < 1 || blocks > 0x7fffffffL) return hipErrorInvalidValue;
+    const BatchPtr<const Tin> in{(const Tin*)a.in, a.in_tab, a.bs_in};
+    const BatchPtr<Tout> out{(Tout*)a.out, a.out_tab, a.bs_out};
+    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(C::NT), C::lds(), a.stream, in, out, a.nx, (T)a.scale,
+                       (const T*)a.tables, a.done, a.nplanes, a.batch, a.reset);
+    return hipGetLastError();
+}
+
+// Columns of a wave tile: 16 hold a 128-byte row segment; a launch whose
+// 16-column tiles leave half the CUs without a block takes 8 (the same bits).
+template <typename Tin, typename Tout, typename T, int LOGN>
+static hipError_t yaxis_wave(const AxisArgs& a) {
+    const long tiles16 = (long)((a.nx + 15) / 16) * a.nplanes * a.batch;
+    return tiles16 <= 128 ? yaxis_wave_k<Tin, Tout, T, LOGN, 8>(a) : yaxis_wave_k<Tin, Tout, T, LOGN, 16>(a);
+}
+
+template <typename Tin, typename Tout, typename T, int LOGN, int TILE>
 static hipError_t yaxis_tile(const AxisArgs& a) {
-    if (a.kind == kDst) return yaxis_k<Tin, Tout, T, LOGN, kDst, TILE>(a);
+    if constexpr (LOGN != 9 && !(LOGN == 8 && TILE == 16))   // else yaxis_wave
+        if (a.kind == kDst) return yaxis_k<Tin, Tout, T, LOGN, kDst, TILE>(a);
     if constexpr (std::is_same_v<Tin, T> && std::is_same_v<Tout, T>) {
         if (a.kind == kRdftFwd) return yaxis_k<Tin, Tout, T, LOGN, kRdftFwd, TILE>(a);
         if (a.kind == kRdftInv) return yaxis_k<Tin, Tout, T, LOGN, kRdftInv, TILE>(a);
@@ -380,6 +481,14 @@ template <typename Tin, typename Tout, typename T, int LOGN>
 static hipError_t yaxis_t(const AxisArgs& a) {
     const int tile = a.tile ? a.tile : default_tile_y<T>(LOGN, a.nx);
     if (!tile_ok<T>(LOGN, tile)) return hipErrorInvalidValue;
+    // DST columns a lane group to a pair: all of N = 512, and of N = 256 the
+    // 16-column tiles, which 2-D plans ask for (planes of a cube fill the chip,
+    // where wider tiles are as fast, and FP32 ones share their bits with
+    // plane_reg_kernel)
+    if constexpr (LOGN == 9)
+        if (a.kind == kDst) return yaxis_wave<Tin, Tout, T, LOGN>(a);
+    if constexpr (LOGN == 8)
+        if (a.kind == kDst && tile == 16) return yaxis_wave<Tin, Tout, T, LOGN>(a);
     if (tile == 16) return yaxis_tile<Tin, Tout, T, LOGN, 16>(a);
     if constexpr (LOGN >= 5) {
         if constexpr (tile_lds_bytes(LOGN, 32, sizeof(T)) <= kLdsBytes)

@@ -388,6 +388,34 @@ __device__ __forceinline__ T lane_scan_incl(T v) {
     return v;
 }
 
+// v of another lane by DPP control CTRL, 0 where that lane is none or the row
+// of 16 is not in ROWS.
+template <int CTRL, int ROWS, typename T>
+__device__ __forceinline__ T dpp_or_zero(T v) {
+    if constexpr (sizeof(T) == 8) {
+        const long long b = __builtin_bit_cast(long long, v);
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+        return __builtin_bit_cast(T, (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+    } else {
+        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, ROWS, 0xf, false));
+    }
+}
+
+// Inclusive scan over each half (L = 32) or all (64) of the wavefront: rows of
+// 16 by row_shr, then lane 15's sum into the next row (rows 1 and 3) and lane
+// 31's into rows 2 and 3.
+template <int L, typename T>
+__device__ __forceinline__ T wave_scan_incl(T v) {
+    v += dpp_or_zero<0x111, 0xf>(v);
+    v += dpp_or_zero<0x112, 0xf>(v);
+    v += dpp_or_zero<0x114, 0xf>(v);
+    v += dpp_or_zero<0x118, 0xf>(v);
+    v += dpp_or_zero<0x142, 0xa>(v);
+    if constexpr (L == 64) v += dpp_or_zero<0x143, 0xc>(v);
+    return v;
+}
+
 // Orders the LDS accesses of one wavefront across lanes.  A job's lanes lie in
 // one wavefront, whose LDS instructions execute in issue order, so only the
 // compiler's code motion has to be fenced.
@@ -773,6 +801,158 @@ __device__ __forceinline__ void dst_pairs128(T* __restrict__ lds, const Lane& L,
     }
     wave_lds_sync();
 }
+
+// ---------------------------------------------------------------------------
+// The DST-I of N = 256 or 512 points with N/8 lanes to a pair of pencils.
+//
+// The packed FFT is 8 x 8 x R, R = N/64: L = N/8 lanes hold eight points each,
+// so a lane's work between exchanges is one dft<8>.  (As 16 lanes of a 32-point
+// and two 16-point DFTs, a pass of 511 x 511 FP64 points took 14.7 us: 32 blocks of
+// two wavefronts, each a chain of some 1600 FP64 instructions with nothing
+// beside it.)
+//   j = t + L j2, t = p + R n;  k = k2 + 8 (m + 8 q), m = s + R e
+//   1. DFT over j2 -> k2, times w_N^{t k2}       lane t -> lanes (k2, p)
+//   2. DFT over n  -> m,  times w_L^{p m}        lane (k2, p) -> (k2, s)
+//   3. DFT over p  -> q                          Z_k, then step 3 of pencil_pairs
+// Exchanges go through the pencils' own slots.  The swizzles are linear over the
+// bits of the index, chosen so that 32 consecutive lanes read and 16 write
+// distinct banks of eight bytes:
+//   exchange 1:  slot L k2 + (t ^ x),                 x = R k2 mod 32
+//   exchange 2:  slot L k2 + ((8 p + (m ^ p)) ^ x)
+//   Z:           posZ: bits 4, 5, 6 of k into bits 2, 1, 0
+//   outputs:     sigma: bits 4, 5, 6 of j into bits 0, 1, 2
+// ---------------------------------------------------------------------------
+template <typename T, int LOGN>
+struct WaveDst {
+    static constexpr int N = 1 << LOGN, L = N / 8, R = L / 8, E = 8 / R;
+    static_assert(L == 32 || L == 64, "half or all of a wavefront");
+    T twr[8], twi[8];   // w_N^{t k}
+    T ur[8], ui[8];     // w_L^{(t mod R) m}
+    T sp[8];            // sin(pi (t + L j)/N) + 1/2
+    __device__ static constexpr int posZ(int k) {
+        return k ^ ((k >> 6) & 1) ^ (((k >> 5) & 1) << 1) ^ (((k >> 4) & 1) << 2);
+    }
+    __device__ static constexpr int sigma(int j) { return j ^ ((j >> 4) & 7); }
+    // slot of output point m (as PencilIO<kDst>::out)
+    __device__ static constexpr int out(int m) { return sigma(m + 1); }
+    // tables as DstLane::init
+    __device__ __forceinline__ void init(const T* __restrict__ tables, const int t) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            sp[k] = tables[2 * N + t + L * k];
+            if (k == 0) continue;
+            twr[k] = tables[t * k];
+            twi[k] = tables[N + t * k];
+            ur[k] = tables[8 * (t % R) * k];
+            ui[k] = tables[N + 8 * (t % R) * k];
+        }
+    }
+
+    // The pencils a and b (N slots each, points in natural order from slot 1,
+    // slot 0 finite), transformed in place by the L lanes t.
+    __device__ __forceinline__ void pair(T* __restrict__ a, T* __restrict__ b, const T scale, const int t) const {
+        T yr[8], yi[8];
+        const int m0 = (N - t) & (N - 1);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {   // N - (t + L j) = L - t + L (7 - j) but for t = j = 0
+            const int o = t + L * j, n = j == 0 ? m0 : L - t + L * (7 - j);
+            const T a0 = a[o], a1 = a[n], b0 = b[o], b1 = b[n];
+            yr[j] = fma(sp[j], a0 + a1, -a1);
+            yi[j] = fma(sp[j], b0 + b1, -b1);
+        }
+        dft<8>(yr, yi);
+#pragma unroll
+        for (int k = 1; k < 8; ++k) rotate(yr[k], yi[k], twr[k], twi[k]);
+        wave_lds_sync();
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int o = L * k + (t ^ (R * k & 31));
+            a[o] = yr[k];
+            b[o] = yi[k];
+        }
+        wave_lds_sync();
+        const int k2 = t / R, p = t % R, x = R * k2 & 31;
+#pragma unroll
+        for (int n = 0; n < 8; ++n) {
+            const int o = L * k2 + p + ((R * n & 31) ^ x) + (R * n & 32);
+            yr[n] = a[o];
+            yi[n] = b[o];
+        }
+        dft<8>(yr, yi);
+#pragma unroll
+        for (int m = 1; m < 8; ++m) rotate(yr[m], yi[m], ur[m], ui[m]);
+        wave_lds_sync();
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            const int o = L * k2 + ((8 * p + (m ^ p)) ^ x);
+            a[o] = yr[m];
+            b[o] = yi[m];
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int e = 0; e < E; ++e) {   // lane (k2, s = p)
+            T vr[R], vi[R];
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                const int o = L * k2 + ((8 * q + ((p + R * e) ^ q)) ^ x);
+                vr[q] = a[o];
+                vi[q] = b[o];
+            }
+            dft<R>(vr, vi);
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                yr[R * e + q] = vr[q];
+                yi[R * e + q] = vi[q];
+            }
+        }
+        wave_lds_sync();
+        const int z = posZ(k2 + 8 * p);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+#pragma unroll
+            for (int q = 0; q < R; ++q) {   // posZ of the constant part: its own bits, and 5 and 6 into 1 and 0
+                const int c = 8 * R * e + 64 * q, o = (z ^ (posZ(c) ^ c)) + c;
+                a[o] = yr[R * e + q];
+                b[o] = yi[R * e + q];
+            }
+        }
+        wave_lds_sync();
+        // even outputs directly, odd ones by prefix sum; lane t owns k = 4 t + i
+        const T hs = T(0.5) * scale;
+        T ae[4], ao[4], be[4], bo[4];
+        T runA = T(0), runB = T(0);
+        const int zk = posZ(4 * t), z0 = posZ((N - 4 * t) & (N - 1)), zn = posZ(4 * (2 * L - 1 - t));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int k = zk ^ i, n = i == 0 ? z0 : zn ^ (4 - i);
+            const T zkr = a[k], zki = b[k], znr = a[n], zni = b[n];
+            ae[i] = zni - zki;
+            be[i] = zkr - znr;
+            T dA = zkr + znr, dB = zki + zni;
+            if (i == 0 && t == 0) {
+                dA *= T(0.5);
+                dB *= T(0.5);
+            }
+            runA += dA;
+            runB += dB;
+            ao[i] = runA;
+            bo[i] = runB;
+        }
+        const T offA = wave_scan_incl<L>(runA) - runA, offB = wave_scan_incl<L>(runB) - runB;
+        wave_lds_sync();
+        const int sw = (t >> 1) & 7;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {   // sigma(8 t + c) = 8 t + (c ^ sw)
+            const bool k0 = i == 0 && t == 0;
+            const int e = 8 * t + ((2 * i) ^ sw), o = 8 * t + ((2 * i + 1) ^ sw);
+            a[e] = k0 ? T(0) : ae[i] * hs;
+            b[e] = k0 ? T(0) : be[i] * hs;
+            a[o] = (ao[i] + offA) * hs;
+            b[o] = (bo[i] + offB) * hs;
+        }
+        wave_lds_sync();
+    }
+};
 
 // ---------------------------------------------------------------------------
 // Constant-coefficient cyclic reduction along z for one (kx,ky) mode.
