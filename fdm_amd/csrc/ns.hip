@@ -8,8 +8,8 @@
 //   v  i in [0,nz+1], k in [-1,ny+1], j in [0,nx+1]
 //   w  i in [-1,nz+1], k in [0,ny+1], j in [0,nx+1]
 //   p  [0,n+1]^3;  x, RHS [1,n]^3;  F j in [0,nx];  G k in [0,ny];  H i in [0,nz]
-// A step is 4 kernels plus the Poisson solve on one stream; from the third
-// step on it is replayed from a hipGraph captured from one step.
+// A step is 4 kernels plus the Poisson solve on one stream; single FP64 steps of
+// small grids are replayed from a hipGraph captured from one step.
 // Arithmetic is FP64 except inside an FP32+refine Poisson solve.
 #include <hip/hip_runtime.h>
 
@@ -309,6 +309,8 @@ __global__ void ns_maxabs_final_kernel(const double* __restrict__ part, double* 
 
 }  // namespace
 
+constexpr long kReplayPoints = 1L << 17;   // grids whose single FP64 steps are replayed from a graph
+
 struct fdmgpu_ns_t {
     int device = 0;
     Grid g{};
@@ -321,7 +323,6 @@ struct fdmgpu_ns_t {
     hipGraphExec_t exec = nullptr;
     long steps = 0;
     bool warm_ok = false;          // x holds the pressure of the previous step (a field upload clears it)
-    bool use_graph = true;
     int* d_bad = nullptr;          // set on the device when a projection misses its tolerance (sticky)
     double* d_max = nullptr;       // maxabs: 9 x kMaxabsBlocks partial maxima, then the 9 results
     hipEvent_t ev_phase[5] = {};   // timed steps: the bounds of the four phases
@@ -482,10 +483,19 @@ int fdmgpu_ns_step(fdmgpu_ns N, int count, void* stream) {
     hipStream_t s = N->cap;
     NS_HIPCHK(hipEventRecord(N->ev_in, user));
     NS_HIPCHK(hipStreamWaitEvent(s, N->ev_in, 0));
+    // A replayed step leaves the GPU idle for about 8 us before its first kernel,
+    // while the host enqueues a step's launches (28 us for 7, 60 for 14) in less
+    // time than all but the smallest grids' steps run; steps behind others hide
+    // even that.  Replayed / one by one, us a step: 127^3 FP32+refine 194 / 188,
+    // FP64 127 / 121; 31^3 FP64 40 / 30 in calls of ten steps, 59 / 67 in calls of one;
+    // 63^3 FP64 in calls of one 69 / 64.
+    const bool replay = count == 1 && N->plan->precision == FDMGPU_F64 &&
+                        (long)N->g.nx * N->g.ny * N->g.nz <= kReplayPoints;
     for (int c = 0; c < count; c++) {
-        // eager for the first two steps (allocations, warm-up) and for a step
-        // whose solve starts from zero after a field upload; replayed after
-        if (!N->use_graph || N->steps < 2 || !N->warm_ok) {
+        // Launched one by one, except a single short step of a small grid (below).
+        // The first two steps (allocations, warm-up) and a step whose solve starts
+        // from zero after a field upload are never replayed.
+        if (!replay || N->steps < 2 || !N->warm_ok) {
             int rc = ns_enqueue_step(N, s);
             if (rc) return rc;
         } else {
