@@ -146,19 +146,34 @@ __global__ __launch_bounds__(256) void zcr_kernel(const BatchPtr<Ts> data, const
     const bool valid = m < plane;
     const long mm = valid ? m : 0;
     const auto base = as_global(data(p) + mm);
-    const int ky = (int)(mm / nx), kx = (int)(mm - (long)ky * nx);
+    const int ky = (int)((unsigned)mm / (unsigned)nx), kx = (int)mm - ky * nx;
 
     T v[C];
-#pragma unroll
-    for (int r = 0; r < C; ++r) {
-        const int row = c * C + r;
-        // branch-free: the row is clamped into the field and the value
-        // selected, so all C loads are in flight together
-        const T x = (T)base[(long)(row < NQ - 1 ? row : NQ - 2) * plane];
-        v[r] = (valid && row < NQ - 1) ? x * gamma : T(0);
-    }
     CrLevels<T, Q> L;
-    cr_levels<T, Q>(L, b, (T)lmx[kx] + (T)lmy[ky]);
+    // branch-free: a row is clamped into the field and its value selected, so
+    // all C loads are in flight together
+    auto row_at = [&](int r) { return base[(long)(c * C + r < NQ - 1 ? c * C + r : NQ - 2) * plane]; };
+    auto put = [&](int r, T x) { v[r] = (valid && c * C + r < NQ - 1) ? x * gamma : T(0); };
+    if constexpr (sizeof(Ts) == sizeof(T)) {
+        // The mode's eigenvalues ahead of the rows: loads return in order, so the
+        // levels are computed while the rows are in flight (31^3 FP64 14.2 -> 13.9 us
+        // a solve, 63^3 20.1 -> 19.9; rows of floats, converted as they come,
+        // measured no faster so).
+        const T lam = (T)lmx[kx] + (T)lmy[ky];
+        __builtin_amdgcn_sched_barrier(0);
+        T raw[C];
+#pragma unroll
+        for (int r = 0; r < C; ++r) raw[r] = row_at(r);
+        __builtin_amdgcn_sched_barrier(0);
+        cr_levels<T, Q>(L, b, lam);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < C; ++r) put(r, raw[r]);
+    } else {
+#pragma unroll
+        for (int r = 0; r < C; ++r) put(r, (T)row_at(r));
+        cr_levels<T, Q>(L, b, (T)lmx[kx] + (T)lmy[ky]);
+    }
     cr_dirichlet_lanes<T, Q, GM>(v, L, lane, s, c);
 
     if (valid) {
@@ -210,19 +225,34 @@ __global__ __launch_bounds__((64 * ZcrStripCfg<Q, CR>::G * S)) void zcr_strip_ke
     const bool valid = m < plane;
     const long mm = valid ? m : 0;
     const auto base = as_global(data(p) + mm);
-    const int ky = (int)(mm / nx), kx = (int)(mm - (long)ky * nx);
+    const int ky = (int)((unsigned)mm / (unsigned)nx), kx = (int)mm - ky * nx;
 
     T v[C];
-#pragma unroll
-    for (int r = 0; r < C; ++r) {
-        const int row = c * C + r;
-        // branch-free: the row is clamped into the field and the value
-        // selected, so all C loads are in flight together
-        const T x = (T)base[(long)(row < NQ - 1 ? row : NQ - 2) * plane];
-        v[r] = (valid && row < NQ - 1) ? x * gamma : T(0);
-    }
     CrLevels<T, Q> L;
-    cr_levels<T, Q>(L, b, (T)lmx[kx] + (T)lmy[ky]);
+    // branch-free: a row is clamped into the field and its value selected, so
+    // all C loads are in flight together
+    auto row_at = [&](int r) { return base[(long)(c * C + r < NQ - 1 ? c * C + r : NQ - 2) * plane]; };
+    auto put = [&](int r, T x) { v[r] = (valid && c * C + r < NQ - 1) ? x * gamma : T(0); };
+    if constexpr (sizeof(Ts) == sizeof(T)) {
+        // The mode's eigenvalues ahead of the rows: loads return in order, so the
+        // levels are computed while the rows are in flight (31^3 FP64 14.2 -> 13.9 us
+        // a solve, 63^3 20.1 -> 19.9; rows of floats, converted as they come,
+        // measured no faster so).
+        const T lam = (T)lmx[kx] + (T)lmy[ky];
+        __builtin_amdgcn_sched_barrier(0);
+        T raw[C];
+#pragma unroll
+        for (int r = 0; r < C; ++r) raw[r] = row_at(r);
+        __builtin_amdgcn_sched_barrier(0);
+        cr_levels<T, Q>(L, b, lam);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < C; ++r) put(r, raw[r]);
+    } else {
+#pragma unroll
+        for (int r = 0; r < C; ++r) put(r, (T)row_at(r));
+        cr_levels<T, Q>(L, b, (T)lmx[kx] + (T)lmy[ky]);
+    }
 
     // forward reduction inside the chunk
     T toRight = T(0), toLeft = T(0);
