@@ -267,6 +267,12 @@ __device__ __forceinline__ int opaque(int x) {
     return x;
 }
 
+// The same for a value computed anew where it stands (never hoisted or shared).
+__device__ __forceinline__ int opaque_volatile(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
 // Plane of rows with pitch P; element (row, col) at row*P + col + f(row).
 // Pencils are rows (x pass) or columns (y pass).
 template <int P, int N1, bool ALONG_X>
@@ -298,42 +304,6 @@ struct PlaneLayout {
         } else {
             return opaque(lv * P + Sw::f(lv) + pencil) + (DP + cp * P);
         }
-    }
-};
-
-// FP64 plane of N = 128 (N1 = 8, 64 jobs per pass): no row swizzle, a pitch
-// P = 2 (mod 32) slots, and jobs dealt to pencils out of order so that both
-// the b64 reads (32 eight-byte banks per half-wavefront: 4 jobs) and the b64
-// writes (16 per quarter-wavefront: 2 jobs) of either pass are
-// conflict-free.  A job's 8 lanes touch slots 8m + (t ^ c) of its pencils
-// (m fixed or t-dependent): along a row those are 8 distinct banks, down a
-// column rows r with 2r mod 32 spread over 8 distinct even banks.  So
-//   x pass (pencils = rows): a job takes rows r and r + 1 (r even: the
-//     second pencil one row on, an offset a ds instruction carries); the 4
-//     jobs of a half-wavefront take r = e, e+4, e+8, e+12 (2r = 2e + 0, 8,
-//     16, 24 mod 32), the 2 of a quarter-wavefront rows 4 apart (8 banks
-//     apart mod 16);
-//   y pass (pencils = columns): a job takes columns c and c + 64; the 4 jobs
-//     of a half-wavefront take c, c+1, c+16, c+17 (odd/even and low/high
-//     halves of the 32 banks), the 2 of a quarter-wavefront c, c+1.
-// 128 rows of 130 slots: 133 KB for a FP64 plane (the swizzled layout's
-// pitch 136 takes 139 KB).
-template <int P, bool ALONG_X>
-struct PlaneLayoutB64 {
-    static_assert(P % 32 == 2, "pitch 2 mod 32");
-    __device__ static constexpr int pencil(int jj) {
-        const int q = jj >> 2, i = jj & 3;
-        return ALONG_X ? 16 * (q >> 1) + 2 * (q & 1) + 4 * i : 32 * (q >> 3) + 2 * (q & 7) + (i & 1) + 16 * (i >> 1);
-    }
-    static constexpr int pair_delta(int jobs) { return ALONG_X ? 1 : jobs; }
-    __device__ static constexpr int at(int row, int col) { return row * P + col; }
-    __device__ static constexpr int addr(int pencil, int slot) {
-        return ALONG_X ? at(pencil, slot) : at(slot, pencil);
-    }
-    template <int DP>
-    __device__ static int addr_split(int pencil, int lv, int cp) {
-        if constexpr (ALONG_X) return opaque(pencil * P + lv) + (DP * P + cp);
-        else return opaque(lv * P + pencil) + (DP + cp * P);
     }
 };
 
@@ -402,8 +372,14 @@ __device__ __forceinline__ T dpp_or_zero(T v) {
     }
 }
 
-// Inclusive scan over each half (L = 32) or all (64) of the wavefront: rows of
-// 16 by row_shr, then lane 15's sum into the next row (rows 1 and 3) and lane
+// v of the lane's neighbour t ^ 1 (quad_perm 1, 0, 3, 2).
+template <typename T>
+__device__ __forceinline__ T lane_xor1(T v) {
+    return dpp_or_zero<0xb1, 0xf>(v);
+}
+
+// Inclusive scan over each row (L = 16), half (32) or all (64) of the wavefront:
+// rows of 16 by row_shr, then lane 15's sum into the next row (rows 1 and 3) and lane
 // 31's into rows 2 and 3.
 template <int L, typename T>
 __device__ __forceinline__ T wave_scan_incl(T v) {
@@ -411,7 +387,7 @@ __device__ __forceinline__ T wave_scan_incl(T v) {
     v += dpp_or_zero<0x112, 0xf>(v);
     v += dpp_or_zero<0x114, 0xf>(v);
     v += dpp_or_zero<0x118, 0xf>(v);
-    v += dpp_or_zero<0x142, 0xa>(v);
+    if constexpr (L >= 32) v += dpp_or_zero<0x142, 0xa>(v);
     if constexpr (L == 64) v += dpp_or_zero<0x143, 0xc>(v);
     return v;
 }
@@ -651,9 +627,7 @@ __device__ __forceinline__ void dst_pairs(T* __restrict__ lds, const DstLane<T, 
 // H[c] + (8 slots) * (constant part of m), H[c] = offset of slot t ^ c: one
 // add per distinct (base, c) where the generic path computes the slot and
 // its swizzle per access.
-// B64: the plane is a PlaneLayoutB64 (no row swizzle, jobs dealt to pencils
-// by its pencil()) instead of a swizzled PlaneLayout.
-template <typename T, int P, int JOBS, int NT, bool COLS, typename Lane = DstLane<T, 7>, bool B64 = false>
+template <typename T, int P, int JOBS, int NT, bool COLS, typename Lane = DstLane<T, 7>>
 __device__ __forceinline__ void dst_pairs128(T* __restrict__ lds, const Lane& L, const T scale,
                                              const int tid) {
     using S = DstShape<7>;
@@ -666,17 +640,13 @@ __device__ __forceinline__ void dst_pairs128(T* __restrict__ lds, const Lane& L,
     constexpr int PBO = COLS ? JOBS * ES : JOBS * P * ES;   // pencil g + JOBS (f(g + JOBS) = f(g))
     static_assert(JOBS % N1 == 0, "swizzle period");
     const int t = tid & (N1 - 1);
-    const int g = [&] {
-        if constexpr (B64) return PlaneLayoutB64<P, !COLS>::pencil(tid / N1);
-        else return tid / N1;
-    }();
+    const int g = tid / N1;
     char* const base = reinterpret_cast<char*>(lds);
-    auto fsw = [](int r) { return B64 ? 0 : Sw::f(r); };
-    auto rowb = [&](int r) { return COLS ? (r * P + fsw(r)) * ES : r * ES; };   // slot r of pencil 0
+    auto rowb = [&](int r) { return COLS ? (r * P + Sw::f(r)) * ES : r * ES; };   // slot r of pencil 0
     int H[N1];
 #pragma unroll
     for (int c = 0; c < N1; ++c) H[c] = opaque(rowb(t ^ c));
-    const int pb = COLS ? g * ES : (g * P + fsw(g)) * ES;
+    const int pb = COLS ? g * ES : (g * P + Sw::f(g)) * ES;
     const int b0 = opaque(pb), b1 = opaque(pb + ROW8 * t), b2 = opaque(pb + 2 * ROW8 * t),
               b3 = opaque(pb + ROW8 * (15 - t));
     // the slots outside the 8m + (t ^ c) form: N - t (step 1, j = t) and the
@@ -953,6 +923,178 @@ struct WaveDst {
         wave_lds_sync();
     }
 };
+
+// ---------------------------------------------------------------------------
+// pencil_pairs<KIND> for all rows (COLS false) or columns (COLS true) of a 128 x
+// 128 plane, 16 lanes of eight points to a pair of pencils: 1024 threads, one job
+// each.
+//
+// The packed FFT is 8 x 8 x 2 (WaveDst with L = 16, R = 2); the radix-2 stage
+// stays in registers, its operands exchanged with the neighbouring lane by DPP,
+// so a pass makes the four trips through LDS that pencil_pairs makes with 8
+// lanes of 16 points, with half the registers a thread and twice the wavefronts
+// to hide their latency.
+//
+// Layout: rows of pitch P = 129, no swizzle; a job takes pencils q and q + 1, the
+// two jobs of 32 lanes pencils 16 apart.  In every access a job's 16 lanes take
+// slots distinct mod 16, and 16 rows or columns are 16 banks mod 32, so reads
+// (32 lanes) and writes (16 of eight bytes) are free of conflicts in both passes.
+// Slots: exchange 1 at 16 k2 + (t ^ 2 k2); Z by posZ (bits 4, 5 of k into bits
+// 0, 1, bit 6 into bit 3), where the periodic kinds leave their outputs; DST
+// outputs by sigma, as DstShape<7>.
+// ---------------------------------------------------------------------------
+constexpr int kWidePitch = 129;
+__device__ constexpr int wide_posZ(int k) { return k ^ ((k >> 4) & 3) ^ (((k >> 6) & 1) << 3); }
+// slot that holds output point m (as PencilIO::out)
+template <int KIND>
+__device__ constexpr int wide_out(int m) {
+    return KIND == kDst ? DstShape<7>::sigma(m + 1) : wide_posZ(m);
+}
+
+// Lane t's constants in LDS (held in registers they would spill what a streaming
+// kernel prefetches): the shifted sines, then w_128^{t k} as [k - 1][t] pairs.
+template <typename T>
+struct Wide128Lane {
+    static constexpr int kValues = 128 + 2 * 16 * 7;
+    const T* sl;
+    const T* tl;
+    __device__ static void fill(const T* __restrict__ tables, T* lds, const int tid, const int nt) {
+        for (int m = tid; m < 128; m += nt) lds[m] = tables[256 + m];
+        for (int m = tid; m < 16 * 7; m += nt) {
+            const int tk = (m & 15) * (m / 16 + 1);
+            lds[128 + 2 * m] = tables[tk];
+            lds[128 + 2 * m + 1] = tables[128 + tk];
+        }
+    }
+    __device__ __forceinline__ Wide128Lane(const T* lds, const int t) : sl(lds + t), tl(lds + 128 + 2 * t) {}
+};
+
+template <int KIND, bool COLS, typename T>
+__device__ __forceinline__ void wide_pairs128(T* __restrict__ lds, const Wide128Lane<T>& L, const T scale,
+                                              const int tid) {
+    constexpr int N = 128, P = kWidePitch, ES = (int)sizeof(T);
+    constexpr int SB = (COLS ? P : 1) * ES, DB = (COLS ? 1 : P) * ES;   // bytes from slot to slot, pencil to pencil
+    constexpr bool HI = 127 * SB + DB > 65535;   // more than a ds instruction's offset carries
+    const int t = tid & 15, p = t & 1, k2 = t >> 1, g = tid >> 4;
+    const int q = 32 * (g >> 4) + 2 * ((g >> 1) & 7) + 16 * (g & 1);
+    const int pb = opaque(q * DB), ph = HI ? opaque(pb + 64 * SB) : pb;
+    char* const mem = reinterpret_cast<char*>(lds);
+    // slot `lane` + c of pencil q, c a compile-time constant
+    auto at = [&](const int lane, const int c) -> T* {
+        return reinterpret_cast<T*>(mem + (HI && c >= 64 ? ph + lane * SB + (c - 64) * SB : pb + lane * SB + c * SB));
+    };
+    auto B = [](T* a) -> T& { return *reinterpret_cast<T*>(reinterpret_cast<char*>(a) + DB); };
+
+    T yr[8], yi[8];
+    const int m0 = (N - t) & (N - 1);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        T* a = at(t, 16 * j);
+        const T a0 = *a, b0 = B(a);
+        if constexpr (KIND == kRdftFwd) {
+            yr[j] = a0;
+            yi[j] = b0;
+        } else {
+            T* n = j == 0 ? at(m0, 0) : at(16 - t, 16 * (7 - j));
+            const T a1 = *n, b1 = B(n);
+            if constexpr (KIND == kDst) {
+                const T sp = L.sl[16 * j];
+                yr[j] = fma(sp, a0 + a1, -a1);
+                yi[j] = fma(sp, b0 + b1, -b1);
+            } else {   // points t + 16 j below N/2, then above; 0 and N/2 stand alone
+                const bool edge = (j == 0 || j == 4) && t == 0;
+                yr[j] = edge ? T(0.5) * a0 : j < 4 ? T(0.5) * (a0 + b1) : T(0.5) * (a1 - b0);
+                yi[j] = edge ? T(-0.5) * b0 : j < 4 ? T(0.5) * (a1 - b0) : T(-0.5) * (a0 + b1);
+            }
+        }
+    }
+    dft<8>(yr, yi);
+#pragma unroll
+    for (int k = 1; k < 8; ++k) rotate(yr[k], yi[k], L.tl[32 * (k - 1)], L.tl[32 * (k - 1) + 1]);
+    wave_lds_sync();
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        T* a = at(t ^ (2 * k), 16 * k);
+        *a = yr[k];
+        B(a) = yi[k];
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+        T* a = at(16 * k2 + p + 2 * (n ^ k2), 0);
+        yr[n] = *a;
+        yi[n] = B(a);
+    }
+    dft<8>(yr, yi);
+    // lane p: the odd points' twiddles w_16^m, then self + other (p = 0) or other - self
+    const T sg = p ? T(-1) : T(1);
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+        if (m > 0) rotate(yr[m], yi[m], p ? (T)cos32(2 * m) : T(1), p ? (T)-sin32(2 * m) : T(0));
+        yr[m] = fma(sg, yr[m], lane_xor1(yr[m]));
+        yi[m] = fma(sg, yi[m], lane_xor1(yi[m]));
+    }
+    wave_lds_sync();
+    const int z = k2 + 8 * p;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {   // k = k2 + 8 m + 64 p
+        T* a = at((z ^ ((m >> 1) + 8 * (m & 1))) + 64 * p, 16 * (m >> 1));
+        *a = KIND == kRdftInv ? yr[m] * scale : yr[m];      // x^a = Re Y, x^b = -Im Y
+        B(a) = KIND == kRdftInv ? -yi[m] * scale : yi[m];
+    }
+    wave_lds_sync();
+    if constexpr (KIND == kRdftInv) return;
+    const int zk = wide_posZ(4 * t), z0 = wide_posZ((N - 4 * t) & (N - 1)), zn = wide_posZ(4 * (31 - t));
+    if constexpr (KIND == kRdftFwd) {
+        // split the packed spectra: lane t owns k = 4 t + i and the mirrors N - k
+        // (k = 0: the Nyquist slot N/2)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool k0 = i == 0 && t == 0;
+            T *k = at(zk ^ i, 0), *n = at(i == 0 ? (t == 0 ? wide_posZ(N / 2) : z0) : zn ^ (4 - i), 0);
+            const T zkr = *k, zki = B(k), znr = *n, zni = B(n);
+            *k = (k0 ? zkr : T(0.5) * (zkr + znr)) * scale;
+            B(k) = (k0 ? zki : T(0.5) * (zki + zni)) * scale;
+            *n = (k0 ? znr : T(0.5) * (zni - zki)) * scale;
+            B(n) = (k0 ? zni : T(0.5) * (zkr - znr)) * scale;
+        }
+        wave_lds_sync();
+        return;
+    }
+    // even outputs directly, odd ones by prefix sum; lane t owns k = 4 t + i
+    const T hs = T(0.5) * scale;
+    T ae[4], ao[4], be[4], bo[4];
+    T runA = T(0), runB = T(0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        T *k = at(zk ^ i, 0), *n = at(i == 0 ? z0 : zn ^ (4 - i), 0);
+        const T zkr = *k, zki = B(k), znr = *n, zni = B(n);
+        ae[i] = zni - zki;
+        be[i] = zkr - znr;
+        T dA = zkr + znr, dB = zki + zni;
+        if (i == 0 && t == 0) {
+            dA *= T(0.5);
+            dB *= T(0.5);
+        }
+        runA += dA;
+        runB += dB;
+        ao[i] = runA;
+        bo[i] = runB;
+    }
+    const T offA = wave_scan_incl<16>(runA) - runA, offB = wave_scan_incl<16>(runB) - runB;
+    wave_lds_sync();
+    const int sw = (t >> 1) & 7;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {   // sigma(8 t + c) = 8 t + (c ^ sw)
+        const bool k0 = i == 0 && t == 0;
+        T *e = at(8 * t + ((2 * i) ^ sw), 0), *o = at(8 * t + ((2 * i + 1) ^ sw), 0);
+        *e = k0 ? T(0) : ae[i] * hs;
+        B(e) = k0 ? T(0) : be[i] * hs;
+        *o = (ao[i] + offA) * hs;
+        B(o) = (bo[i] + offB) * hs;
+    }
+    wave_lds_sync();
+}
 
 // ---------------------------------------------------------------------------
 // Constant-coefficient cyclic reduction along z for one (kx,ky) mode.

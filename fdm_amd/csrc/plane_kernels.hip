@@ -178,42 +178,44 @@ __attribute__((amdgpu_waves_per_eu(PlaneCfg<LOGN>::template waves<T>()))) void p
 
 // ---------------------------------------------------------------------------
 // Streaming plane kernel for FP64 planes of N = 128 (the plain LaplCube<double>
-// solve at 127^3, periodic 128^3).  Such a plane takes 139 KB of LDS, so one
+// solve at 127^3, periodic 128^3).  Such a plane takes 132 KB of LDS, so one
 // block fills a CU; the one-plane-per-block kernel then leaves HBM idle while
 // the block transforms and the CU idle while it loads.  Here a block walks
 // planes q = blockIdx.x, blockIdx.x + gridDim.x, ... (about the same count per
 // block: the grid is sized so), and while plane q is transformed the global
-// loads of its next plane are in flight in registers: the first kStreamSplit
+// loads of its next plane are in flight in registers: the first SPLIT
 // rows of a thread's share issued before the x pass, the rest before the y
 // pass.  After the y pass the outputs are read into registers and, once every
-// wave has read its share, stored kStreamChunk rows at a time between the
+// wave has read its share, stored CHUNK rows at a time between the
 // next plane's staging writes.  (A wave issues its memory instructions in
 // order and stalls while the memory pipeline is full: a whole plane of loads
 // or of stores issued at once held every wave for about 4k cycles per plane,
-// measured with s_memtime stamps.)  The plane sits in LDS in the
-// b64-conflict-free PlaneLayoutB64 (pitch kStreamPitch, jobs dealt to pencils
-// out of order).  Each pencil goes through plane_dst_kernel's transform;
-// results agree with that kernel's to FP64 rounding (2e-14 relative at
-// 127^3), not bitwise.
+// measured with s_memtime stamps.)  Both passes are wide_pairs128's, in its
+// layout; results agree with plane_dst_kernel's to FP64 rounding (2e-14
+// relative at 127^3), not bitwise.  What bounds it: a launch of 32 x 127 planes
+// takes about 250 us, its 1.05 GB at the rate of a large copy 213.
 // ---------------------------------------------------------------------------
-constexpr int kStreamPitch = 130;
-constexpr int kStreamSplit = 16;   // rows (of 32 per thread) prefetched before the x pass
-constexpr int kStreamChunk = 8;    // rows stored between staging writes
+struct StreamCfg {
+    static constexpr int N = 128, NT = 1024, P = kWidePitch;
+    static constexpr int ITER = N * N / NT;      // rows per thread
+    static constexpr int SPLIT = ITER / 2;       // of them prefetched before the x pass
+    static constexpr int CHUNK = ITER / 4;       // rows stored between staging writes
+    using Lane = Wide128Lane<double>;
+    static constexpr size_t lds_bytes() { return sizeof(double) * (size_t)(N * P + Lane::kValues); }
+};
 
 template <int KIND>
-__global__ __launch_bounds__(PlaneCfg<7>::NT) __attribute__((amdgpu_waves_per_eu(2))) void plane_stream_kernel(
+__global__ __launch_bounds__(StreamCfg::NT) __attribute__((amdgpu_waves_per_eu(4))) void plane_stream_kernel(
     const BatchPtr<const double> in, const BatchPtr<double> out, const double sx, const double sy,
     const double* __restrict__ tables, const int nplanes, const int total) {
     constexpr int LOGN = 7;
-    using C = PlaneCfg<LOGN>;
-    using S = DstShape<LOGN>;
+    using C = StreamCfg;
     using IO = PencilIO<KIND, LOGN>;
-    constexpr int P = kStreamPitch;   // conflict-free b64 layout (PlaneLayoutB64)
-    using LX = PlaneLayoutB64<P, true>;
-    using LY = PlaneLayoutB64<P, false>;
+    constexpr int P = C::P;
     constexpr int N = C::N, n = IO::n, o = IO::off, NT = C::NT;
-    constexpr int R = NT / N, ITER = (n + R - 1) / R;
-    static_assert(NT % N == 0, "a block covers whole rows");
+    constexpr int R = NT / N, ITER = C::ITER, SPLIT = C::SPLIT, CHUNK = C::CHUNK;
+    static_assert(NT % N == 0 && ITER == (n + R - 1) / R, "a block covers whole rows");
+    auto at = [](int row, int col) { return row * P + col; };
     const int tid = threadIdx.x;
     int q = blockIdx.x;
     if (q >= total) return;
@@ -227,20 +229,17 @@ __global__ __launch_bounds__(PlaneCfg<7>::NT) __attribute__((amdgpu_waves_per_eu
     // load in bounds or past the buffer's range (which reads 0), stage into
     // the pad column, and store past the range (which is dropped).
     const int x0 = tid & (N - 1), r0 = __builtin_amdgcn_readfirstlane(tid >> LOGN);
-    const int slot0 = opaque(LX::at(ITER * r0 + o, x0 + o));   // element i: slot0 + i P
+    const int slot0 = opaque(at(ITER * r0 + o, x0 + o));   // element i: slot0 + i P
     const int lane_in = (int)((ITER * r0 * n + x0) * sizeof(double));
 
-    // the DST's shifted sines come from an LDS copy behind the plane (the
-    // prefetch takes their registers)
-    using Lane = DstLaneLdsSine<double, LOGN>;
-    double* sines = lds + N * P;
-    Lane L;
-    Lane::fill_sines(tables, sines, tid, NT);
-    L.init(tables, sines, tid & (S::N1 - 1));
+    // the lane constants in LDS behind the plane (the prefetch takes their registers)
+    double* consts = lds + N * P;
+    C::Lane::fill(tables, consts, tid, NT);
+    const C::Lane L(consts, tid & 15);
     if constexpr (KIND == kDst) {   // the dummy row and column stay 0 across planes
         for (int i = tid; i < N; i += NT) {
-            lds[LX::at(0, i)] = 0.0;
-            lds[LX::at(i, 0)] = 0.0;
+            lds[at(0, i)] = 0.0;
+            lds[at(i, 0)] = 0.0;
         }
     }
     double v[ITER];
@@ -260,7 +259,7 @@ __global__ __launch_bounds__(PlaneCfg<7>::NT) __attribute__((amdgpu_waves_per_eu
         for (int i = LO; i < HI; ++i) v[i] = src.load(lane_in, (int)(i * n * sizeof(double)));
     };
     using R0 = std::integral_constant<int, 0>;
-    using RH = std::integral_constant<int, kStreamSplit>;
+    using RH = std::integral_constant<int, SPLIT>;
     using R1 = std::integral_constant<int, ITER>;
     auto load_plane = [&](const int qq) { load_rows(qq, R0{}, R1{}); };
     auto stage_rows = [&](auto loc, auto hic) {
@@ -292,27 +291,18 @@ __global__ __launch_bounds__(PlaneCfg<7>::NT) __attribute__((amdgpu_waves_per_eu
         // the passes' addresses are recomputed per plane from a thread index
         // the compiler cannot hoist out of the loop: kept live across the
         // loop they would take the registers the prefetch needs
-        int t1 = tid;
-        asm volatile("" : "+v"(t1));
-        pencil_pairs<KIND, double, LOGN, N / 2, LX, NT, Lane>(lds, L, sx, t1);   // pencils = rows    (x)
+        wide_pairs128<KIND, false>(lds, L, sx, opaque_volatile(tid));   // pencils = rows    (x)
         __syncthreads();
-        if constexpr (kStreamSplit < ITER)
-            if (qn < total) load_rows(qn, RH{}, R1{});
+        if (qn < total) load_rows(qn, RH{}, R1{});
         __builtin_amdgcn_sched_barrier(0);
-        int t2 = tid;
-        asm volatile("" : "+v"(t2));
-        if constexpr (KIND == kDst)
-            dst_pairs128<double, P, N / 2, NT, true, Lane, true>(lds, L, sy, t2);   // pencils = columns (y)
-        else
-            pencil_pairs<KIND, double, LOGN, N / 2, LY, NT, Lane>(lds, L, sy, t2);
+        wide_pairs128<KIND, true>(lds, L, sy, opaque_volatile(tid));    // pencils = columns (y)
         __syncthreads();
         // store phase: the plane's outputs into registers, then, once every
         // wave has read its share, their global stores interleaved with the
         // next plane's staging (a plane of stores issued at once stalls the
         // wave while the memory pipeline takes them; staged in between, the
         // LDS writes proceed meanwhile)
-        int t3 = tid;
-        asm volatile("" : "+v"(t3));
+        const int t3 = opaque_volatile(tid);
         int p, z;
         split(q, p, z);
         const BufRange<double> dst(wave_uniform(out.uniform(p)) + (long)z * plane_pts, plane_pts * sizeof(double));
@@ -323,7 +313,7 @@ __global__ __launch_bounds__(PlaneCfg<7>::NT) __attribute__((amdgpu_waves_per_eu
         // not have been issued, and count the waits for the prefetch without
         // them: staging would then wait for the stores.)
         const int xo = t3 & (N - 1);
-        const int xs = opaque(IO::out(xo < n ? xo : n - 1));
+        const int xs = opaque(wide_out<KIND>(xo < n ? xo : n - 1));
         const int lane_out = xo < n ? (int)((ITER * r0 * n + xo) * sizeof(double)) : (int)(plane_pts * sizeof(double));
         double o[ITER];
         // the row part of each LDS slot is wave-uniform (scalar arithmetic);
@@ -331,7 +321,7 @@ __global__ __launch_bounds__(PlaneCfg<7>::NT) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
         for (int i = 0; i < ITER; ++i) {
             const int y = ITER * r0 + i, ys = y < n - 1 ? y : n - 1;
-            o[i] = lds[LX::at(IO::out(ys), 0) + xs];
+            o[i] = lds[at(wide_out<KIND>(ys), 0) + xs];
         }
         auto store_rows = [&](auto loc, auto hic) {
             constexpr int LO = decltype(loc)::value, HI = decltype(hic)::value;
@@ -344,11 +334,11 @@ __global__ __launch_bounds__(PlaneCfg<7>::NT) __attribute__((amdgpu_waves_per_eu
         }
         q = qn;
         __syncthreads();   // every wave has read the plane before the next one is staged
-        static_assert(ITER % kStreamChunk == 0, "whole chunks");
-        static_for<0, ITER / kStreamChunk>([&](auto cc) {
+        static_assert(ITER % CHUNK == 0, "whole chunks");
+        static_for<0, ITER / CHUNK>([&](auto cc) {
             constexpr int c = decltype(cc)::value;
-            using Lo = std::integral_constant<int, c * kStreamChunk>;
-            using Hi = std::integral_constant<int, (c + 1) * kStreamChunk>;
+            using Lo = std::integral_constant<int, c * CHUNK>;
+            using Hi = std::integral_constant<int, (c + 1) * CHUNK>;
             store_rows(Lo{}, Hi{});
             stage_rows(Lo{}, Hi{});
         });
@@ -636,9 +626,9 @@ static int device_cus() {
 
 template <int KIND>
 static hipError_t plane_stream_k(const PlaneArgs& a) {
-    using C = PlaneCfg<7>;
+    using C = StreamCfg;
     auto k = plane_stream_kernel<KIND>;
-    const size_t lds = sizeof(double) * (size_t)C::N * (kStreamPitch + 1);   // plane + sine table
+    const size_t lds = C::lds_bytes();
     hipError_t e = allow_lds(k, lds);
     if (e != hipSuccess) return e;
     const long total = (long)a.nplanes * a.batch;
