@@ -529,6 +529,12 @@ int stage_inv(fdmgpu_plan_t* P, void* in, Tab in_tab, void* out, Tab out_tab, in
     return FDMGPU_OK;
 }
 
+// Scale of the z systems' right-hand sides (1 up to rounding for lz = dz n).
+double zcr_gamma(const fdmgpu_plan_t* P) {
+    const double gamma = P->dz * (double)(1 << P->logz) / P->lz;
+    return std::fabs(gamma - 1.0) < 4e-16 ? 1.0 : gamma;
+}
+
 // FP32 plans (LaplCube<float>, LaplRect<float>) eliminate in double: the
 // systems of the lowest modes are nearly singular and an FP32 elimination
 // would lose ~cond * eps there, where the reference's z transforms keep
@@ -539,9 +545,8 @@ int stage_tridiag(fdmgpu_plan_t* P, void* data, Tab data_tab, int count, hipStre
     const long elems = (long)P->nx * P->ny * P->nz;
     if (P->kind == 3) {
         const double b = 1.0 / (P->hz_op * P->hz_op);
-        const double gamma = P->dz * (double)(1 << P->logz) / P->lz;
-        ZcrArgs z{data, (long)P->nx * P->ny, P->nx, P->lmx, P->lmy, b,
-                  std::fabs(gamma - 1.0) < 4e-16 ? 1.0 : gamma, elems, count, s, done, P->periodic != 0,
+        ZcrArgs z{data, (long)P->nx * P->ny, P->nx, P->lmx, P->lmy, b, zcr_gamma(P), elems, count, s, done,
+                  P->periodic != 0,
                   P->precision == FDMGPU_F32, data_tab, P->var.zcr_gmul};
         Timed tm(P, FDMGPU_K_ZCR, s);
         HIPCHK(launch_zcr<T>(P->logz, z));
@@ -570,8 +575,22 @@ int stage_tridiag(fdmgpu_plan_t* P, void* data, Tab data_tab, int count, hipStre
     return FDMGPU_OK;
 }
 
+// Dirichlet cubes that small_cube_kernel solves in one launch, in the default variant.
+bool use_small_cube(const fdmgpu_plan_t* P) {
+    return P->kind == 3 && !P->periodic && P->logx == P->logy && small_cube_ok(P->logx, P->logz) &&
+           P->var.plane == 1 && !P->var.tile_x && !P->var.tile_y && !P->var.zcr_gmul;
+}
+
 template <typename T>
 int solve_plain(fdmgpu_plan_t* P, void* ans, Tab ans_tab, const void* rhs, Tab rhs_tab, int count, hipStream_t s) {
+    if (use_small_cube(P)) {
+        SmallCubeArgs a{rhs, ans, rhs_tab, ans_tab, plan_elems(P), count, P->dx * std::sqrt(2. / P->lx),
+                        P->dy * std::sqrt(2. / P->ly), std::sqrt(2. / P->lx), std::sqrt(2. / P->ly), P->tab_x, P->lmx,
+                        P->lmy, 1.0 / (P->hz_op * P->hz_op), zcr_gamma(P), s};
+        Timed tm(P, FDMGPU_K_OTHER, s);
+        HIPCHK((launch_small_cube<T>(P->logx, P->logz, a)));
+        return FDMGPU_OK;
+    }
     int rc = stage_fwd<T, T>(P, rhs, rhs_tab, ans, ans_tab, count, s, nullptr);
     if (rc) return rc;
     rc = stage_tridiag<T>(P, ans, ans_tab, count, s, nullptr);

@@ -156,6 +156,22 @@ struct ZcrArgs {
     int gmul;             // lanes-per-system multiplier (1 or 2; 0 = 1)
 };
 
+// A whole small Dirichlet cube per block (small_kernels.hip)
+struct SmallCubeArgs {
+    const void* in;
+    void* out;
+    const void* const* in_tab;
+    const void* const* out_tab;
+    long bs;              // elements per problem
+    int batch;
+    double fx, fy, ix, iy;   // scales of the forward and inverse transforms
+    const void* tables;
+    const void* lmx;      // as ZcrArgs
+    const void* lmy;
+    double b, gamma;
+    hipStream_t stream;
+};
+
 struct RowCrArgs {
     void* data;
     int nx, nrows;
@@ -213,6 +229,9 @@ struct PlaneResidArgs {
 
 template <typename Tin, typename Tout, typename T>
 hipError_t launch_plane(int logn, const PlaneArgs& a);
+template <typename T>
+hipError_t launch_small_cube(int logn, int logz, const SmallCubeArgs& a);
+bool small_cube_ok(int logn, int logz);
 // FP32 planes of N = 256 (plane_reg_kernels.hip)
 template <typename Tin, typename Tout>
 hipError_t launch_plane_reg(const PlaneArgs& a);
