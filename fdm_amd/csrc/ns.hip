@@ -322,6 +322,13 @@ struct fdmgpu_ns_t {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     long steps = 0;
+    // the solver's settings of the first replayable step, which later ones keep
+    struct {
+        bool set = false;
+        double rtol = 0;
+        int max_iter = 0;
+        Variant var;
+    } kept;
     bool warm_ok = false;          // x holds the pressure of the previous step (a field upload clears it)
     int* d_bad = nullptr;          // set on the device when a projection misses its tolerance (sticky)
     double* d_max = nullptr;       // maxabs: 9 x kMaxabsBlocks partial maxima, then the 9 results
@@ -386,6 +393,30 @@ int ns_enqueue_step(fdmgpu_ns_t* N, hipStream_t s, hipEvent_t* ev = nullptr) {
     NS_HIPCHK(hipGetLastError());
     NS_HIPCHK(mark(4));
     return FDMGPU_OK;
+}
+
+// A step after the first two, x warm: with the solver settings of the first such
+// step, whether it is replayed or not (fdmgpu_ns_get's contract).
+int ns_enqueue_kept(fdmgpu_ns_t* N, hipStream_t s) {
+    fdmgpu_plan_t* P = N->plan;
+    auto& k = N->kept;
+    if (!k.set) {
+        k.set = true;
+        k.rtol = P->rtol;
+        k.max_iter = P->max_iter;
+        k.var = P->var;
+    }
+    const double rtol = P->rtol;
+    const int max_iter = P->max_iter;
+    const Variant var = P->var;
+    P->rtol = k.rtol;
+    P->max_iter = k.max_iter;
+    P->var = k.var;
+    const int rc = ns_enqueue_step(N, s);
+    P->rtol = rtol;
+    P->max_iter = max_iter;
+    P->var = var;
+    return rc;
 }
 
 // fdmgpu_get_stats on the solver plan reports the last step's pressure solve
@@ -495,13 +526,14 @@ int fdmgpu_ns_step(fdmgpu_ns N, int count, void* stream) {
         // Launched one by one, except a single short step of a small grid (below).
         // The first two steps (allocations, warm-up) and a step whose solve starts
         // from zero after a field upload are never replayed.
-        if (!replay || N->steps < 2 || !N->warm_ok) {
-            int rc = ns_enqueue_step(N, s);
+        const bool later = N->steps >= 2 && N->warm_ok;
+        if (!replay || !later) {
+            int rc = later ? ns_enqueue_kept(N, s) : ns_enqueue_step(N, s);
             if (rc) return rc;
         } else {
             if (!N->exec) {
                 NS_HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed));
-                int rc = ns_enqueue_step(N, s);
+                int rc = ns_enqueue_kept(N, s);
                 hipGraph_t graph = nullptr;
                 hipError_t e = hipStreamEndCapture(s, &graph);
                 if (!rc && e != hipSuccess) rc = FDMGPU_ERR_DEVICE;

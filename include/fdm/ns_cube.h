@@ -29,7 +29,7 @@
 // "Step times (ms): init_bound=.., FGH=.., poisson=.., update_uvwp=..".
 // The phase times are GPU time between the events; the reference's are host
 // wall-clock time of its CPU loops.  verbose == 0: steps are enqueued
-// asynchronously and replayed from a hipGraph (fdmgpu_ns_step).
+// asynchronously (fdmgpu_ns_step).
 #pragma once
 
 #include <array>

@@ -317,8 +317,8 @@ typedef struct fdmgpu_ns_t* fdmgpu_ns;
 int fdmgpu_ns_create(fdmgpu_ns* ns, int solver_precision, int nx, int ny, int nz, double x1, double x2, double y1,
                      double y2, double z1, double z2, double u0, double Re, double dt);
 /* Replaces NSCube::step() (src/ns_cube.cpp:27-62), `count` times, ordered on
- * `stream` (returns after enqueueing); steps from the third on are replayed
- * from a hipGraph of one step. */
+ * `stream` (returns after enqueueing); single steps of small FP64 grids are
+ * replayed from a hipGraph of one step. */
 int fdmgpu_ns_step(fdmgpu_ns ns, int count, void* stream);
 /* Fields with the reference's index ranges (src/ns_cube.h:66-75), x fastest:
  * U [0,nz+1]x[0,ny+1]x[-1,nx+1], V [0,nz+1]x[-1,ny+1]x[0,nx+1],
