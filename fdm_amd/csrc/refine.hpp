@@ -32,6 +32,9 @@ struct ResidualArgs {
     int* bad = nullptr;         // final certification: set to 1 when a problem ends above tol
     int base = 0;               // iters[] as the launch finds it (0, or the previous check's iteration)
     bool first_check = false;   // the solve's first check: done[] is not read, only set
+    bool mark = false;          // 3-D, r32 held back (refine.hip: CheckArgs): after solve 1 mark,
+    bool lazy = false;          //   in the check after solve 2 leave out,
+    bool rewrite = false;       //   and write for marked problems that did not converge
 };
 
 // The residual, its norms and the convergence check, in one launch.  iters[]
