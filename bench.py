@@ -262,10 +262,14 @@ def bytes_per_point(sym: str):
         return 16
     if base == "plane_resid_dst_kernel":       # f, u in; FP32 transformed residual out
         return 8 + sz[a[0]] + 4
+    if base == "plane_reg_kernel":
+        return sz[a[0]] + sz[a[1]] + {0: 0, 1: sz[a[1]], 2: 4}[int(a[2])]
     if base == "xaxis_dst_kernel":
         return sz[a[0]] + sz[a[1]] + (sz[a[1]] if a[4] == "true" else 0)
-    if base == "yaxis_dst_kernel":
+    if base in ("yaxis_dst_kernel", "yaxis_wave_kernel"):
         return sz[a[0]] + sz[a[1]]
+    if base == "small_cube_kernel":
+        return 2 * sz[a[0]]
     if base in ("zcr_strip_kernel", "zcr_kernel", "zcrp_kernel"):
         return 2 * sz[a[0]]
     if base == "residual_tile_kernel":         # f, u in; FP32 residual out when WRITE
