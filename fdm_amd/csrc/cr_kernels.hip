@@ -924,7 +924,7 @@ static hipError_t rowcr_k(const RowCrArgs& a) {
 
 template <typename Ts, typename T>
 static hipError_t rowgtsv_k(const RowCrArgs& a) {
-    const size_t lds = 4 * sizeof(double) * (size_t)a.nx;
+    const size_t lds = 4 * sizeof(T) * (size_t)a.nx;
     hipError_t e = allow_lds(rowgtsv_kernel<Ts, T>, lds);
     if (e != hipSuccess) return e;
     const BatchPtr<Ts> data{(Ts*)a.data, a.data_tab, a.bs};
