@@ -505,7 +505,8 @@ class NSCube:
 
     def set_solver_refine(self, rel_tol: float = 1e-10, max_iter: int = 4):
         """Refinement settings of the FP32+refine pressure solver (fdmgpu_set_refine
-        on the plan of fdmgpu_ns_solver); steps enqueued afterwards use them."""
+        on the plan of fdmgpu_ns_solver).  Steps after the first two whose solve
+        starts warm keep the settings of the first of them."""
         plan = C.c_void_p()
         _check(_lib_handle().fdmgpu_ns_solver(self._h, C.byref(plan)), "NSCube.solver")
         _check(_lib_handle().fdmgpu_set_refine(plan, rel_tol, max_iter), "NSCube.set_solver_refine")

@@ -395,9 +395,13 @@ int ns_enqueue_step(fdmgpu_ns_t* N, hipStream_t s, hipEvent_t* ev = nullptr) {
     return FDMGPU_OK;
 }
 
-// A step after the first two, x warm: with the solver settings of the first such
-// step, whether it is replayed or not (fdmgpu_ns_get's contract).
-int ns_enqueue_kept(fdmgpu_ns_t* N, hipStream_t s) {
+// A step after the first two, x warm.
+bool ns_later(const fdmgpu_ns_t* N) { return N->steps >= 2 && N->warm_ok; }
+
+// Such a step: with the solver settings of the first of them, whether it is
+// replayed, enqueued or timed (the contract of fdmgpu_ns_get and
+// fdmgpu_ns_step_timed).
+int ns_enqueue_kept(fdmgpu_ns_t* N, hipStream_t s, hipEvent_t* ev = nullptr) {
     fdmgpu_plan_t* P = N->plan;
     auto& k = N->kept;
     if (!k.set) {
@@ -412,7 +416,7 @@ int ns_enqueue_kept(fdmgpu_ns_t* N, hipStream_t s) {
     P->rtol = k.rtol;
     P->max_iter = k.max_iter;
     P->var = k.var;
-    const int rc = ns_enqueue_step(N, s);
+    const int rc = ns_enqueue_step(N, s, ev);
     P->rtol = rtol;
     P->max_iter = max_iter;
     P->var = var;
@@ -526,7 +530,7 @@ int fdmgpu_ns_step(fdmgpu_ns N, int count, void* stream) {
         // Launched one by one, except a single short step of a small grid (below).
         // The first two steps (allocations, warm-up) and a step whose solve starts
         // from zero after a field upload are never replayed.
-        const bool later = N->steps >= 2 && N->warm_ok;
+        const bool later = ns_later(N);
         if (!replay || !later) {
             int rc = later ? ns_enqueue_kept(N, s) : ns_enqueue_step(N, s);
             if (rc) return rc;
@@ -564,8 +568,8 @@ int fdmgpu_ns_step_timed(fdmgpu_ns N, double* ms, void* stream) {
     hipStream_t s = N->cap;
     NS_HIPCHK(hipEventRecord(N->ev_in, user));
     NS_HIPCHK(hipStreamWaitEvent(s, N->ev_in, 0));
-    // eager: the same kernels with the same arguments as a replayed step
-    int rc = ns_enqueue_step(N, s, N->ev_phase);
+    // the kernels and arguments of an untimed step
+    int rc = ns_later(N) ? ns_enqueue_kept(N, s, N->ev_phase) : ns_enqueue_step(N, s, N->ev_phase);
     if (rc) return rc;
     N->steps++;
     N->warm_ok = true;

@@ -338,14 +338,15 @@ int fdmgpu_ns_step(fdmgpu_ns ns, int count, void* stream);
  * then returns FDMGPU_ERR_NOT_CONVERGED if any projection so far ended above
  * the solver's tolerance (a flag kept on the device by every step, replayed
  * ones included; it stays set for the rest of the run).  Warm-started
- * projections run inner solves 2 .. max(2, max_iter - 1) of the solver plan's
- * refinement settings as they were when the step was first enqueued. */
+ * projections run inner solves 2 .. max(2, max_iter - 1).  Steps after the
+ * first two whose solve starts warm keep the solver plan's settings (tolerance,
+ * inner solves, variant) of the first of them, however they are launched. */
 int fdmgpu_ns_get(fdmgpu_ns ns, int which, double* host, unsigned long long count);
 int fdmgpu_ns_set(fdmgpu_ns ns, int which, const double* host, unsigned long long count);
 /* Element count and device address of a field (device-side post-processing). */
 int fdmgpu_ns_info(fdmgpu_ns ns, int which, unsigned long long* count, void** device_ptr);
-/* One step, enqueued eagerly (the kernels and arguments of a replayed step,
- * so the fields are bitwise those of fdmgpu_ns_step), with GPU events at the
+/* One step (the kernels and arguments of an untimed one, so the fields are
+ * bitwise those of fdmgpu_ns_step), with GPU events at the
  * bounds of the reference's four phases; waits for it and writes their
  * durations in ms to ms[0..3]: init_bound (lid, ghost layers, pressure
  * boundary), FGH, poisson (right-hand side and the solve), update_uvwp.
