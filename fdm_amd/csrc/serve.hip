@@ -182,7 +182,8 @@ void group_free(fdmgpu_group_t* g) {
         (void)hipFree(b.d_tab);
         if (b.plan) fdmgpu_destroy(b.plan);
     }
-    for (hipEvent_t e : g->joins) (void)hipEventDestroy(e);
+    for (hipEvent_t e : g->joins)   // (the origin stream has none)
+        if (e) (void)hipEventDestroy(e);
     if (g->fork) (void)hipEventDestroy(g->fork);
     if (g->ev_in) (void)hipEventDestroy(g->ev_in);
     if (g->ev_out) (void)hipEventDestroy(g->ev_out);
