@@ -1287,6 +1287,16 @@ int fdmgpu_plan_get_variant(fdmgpu_plan plan, fdmgpu_variant* v) {
     return FDMGPU_OK;
 }
 
+// Memory the runtime does not know: the host stage moves its bytes.  Pinned (or
+// managed, or device) memory is left to the runtime, whose copy of it runs at the
+// link's rate with no thread beside it.
+static bool pageable(const void* p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    return true;
+}
+
 int fdmgpu_solve_host(fdmgpu_plan plan, void* ans, const void* rhs) {
     if (!plan || !ans || !rhs) return FDMGPU_ERR_INVALID_ARG;
     HIPCHK(hipSetDevice(plan->device));
@@ -1302,16 +1312,18 @@ int fdmgpu_solve_host(fdmgpu_plan plan, void* ans, const void* rhs) {
     if (!plan->own) HIPCHK(hipStreamCreateWithFlags(&plan->own, hipStreamNonBlocking));
     char* d_rhs = (char*)plan->stage;
     char* d_ans = plan->precision == FDMGPU_F32_REFINE64 ? d_rhs + bytes : d_rhs;
+    const bool staged_in = bytes >= kStageMin && pageable(rhs), staged_out = bytes >= kStageMin && pageable(ans);
     // a plan that solves once does not pay for setting a stage up
-    if (!plan->host_st && bytes >= kStageMin) plan->host_st = host_stage(plan->device, plan->host_calls > 0);
+    if (!plan->host_st && (staged_in || staged_out))
+        plan->host_st = host_stage(plan->device, plan->host_calls > 0);
     if (plan->host_calls < 2) plan->host_calls++;
-    HostStage* const st = bytes >= kStageMin ? plan->host_st.get() : nullptr;
-    hipError_t e = st ? stage_in(*st, d_rhs, rhs, bytes, plan->own) : hipErrorNotReady;
+    HostStage* const st = plan->host_st.get();
+    hipError_t e = st && staged_in ? stage_in(*st, d_rhs, rhs, bytes, plan->own) : hipErrorNotReady;
     if (e == hipErrorNotReady) e = hipMemcpyAsync(d_rhs, rhs, bytes, hipMemcpyHostToDevice, plan->own);
     HIPCHK(e);
     int rc = solve_device_impl(plan, d_ans, nullptr, d_rhs, nullptr, 1, plan->own);
     if (rc) return rc;
-    e = st ? stage_out(*st, ans, d_ans, bytes, plan->own) : hipErrorNotReady;
+    e = st && staged_out ? stage_out(*st, ans, d_ans, bytes, plan->own) : hipErrorNotReady;
     if (e == hipErrorNotReady) e = hipMemcpyAsync(ans, d_ans, bytes, hipMemcpyDeviceToHost, plan->own);
     HIPCHK(e);
     HIPCHK(hipStreamSynchronize(plan->own));
