@@ -68,3 +68,16 @@ def test_pinned_arrays_pass_the_stage_by():
     assert not threads() & workers                   # ended with the plan
     pin_f.free()
     pin_ans.free()
+
+
+@pytest.mark.parametrize("n,staged", [((63, 63, 63), False), ((127, 63, 63), True)])
+def test_small_arrays_pass_the_stage_by(n, staged):
+    """1.9 MiB, which the runtime copies faster, and 3.8 MiB."""
+    print("[case] host stage from", n, flush=True)
+    s = plan(n)
+    f = np.random.default_rng(1).uniform(-1, 1, n[::-1])
+    ans = np.empty_like(f)
+    s.solve(ans, f)
+    before = threads()
+    s.solve(ans, f)
+    assert len(threads() - before) == (6 if staged else 0)
