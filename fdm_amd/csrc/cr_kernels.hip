@@ -510,13 +510,18 @@ __global__ __launch_bounds__(256) void zcrp_kernel(const BatchPtr<Ts> data, cons
 // One block per row; coefficients and rhs staged in LDS.  Rows of up to 1024
 // points take rowpart_kernel below.
 // Instead of the diagonal a row carries its excess s_j = -D_j - L_j - U_j over the
-// couplings, exact at the start and updated by sums of positive terms (as
-// Grassmann, Taksar and Heyman's elimination does): the near-cancellation of
-// diagonal and couplings, where the lowest modes lose digits, never happens.
-// The arithmetic is FP64 also for FP32 data.
+// couplings, updated by sums of positive terms (as Grassmann, Taksar and Heyman's
+// elimination does): no level adds to the lowest modes' loss of digits where
+// diagonal and couplings nearly cancel.  What D_j's own rounding costs them, as in
+// the reference's matrix, stays: 1e-12 of the lowest mode at 511 x 511 points, 6e-12
+// at 1000 x 511.
+// The arithmetic is FP64 also for FP32 data.  A row is divided by its diagonal once,
+// when it is eliminated: 16 x 511 rows of 4096 points, us a solve, with a division per
+// coupling and level / this: FP64 1015 / 851, FP32+refine 3539 / 3065 (eliminated in
+// FP32, with one inner solve more, 4172).
 // ---------------------------------------------------------------------------
-template <typename Ts>
-__global__ __launch_bounds__(256) void rowcr_kernel(const BatchPtr<Ts> data, const int nx, const int q,
+template <typename Ts, int NT>
+__global__ __launch_bounds__(NT) void rowcr_kernel(const BatchPtr<Ts> data, const int nx, const int q,
                                                     const Ts* __restrict__ lmy, const Ts* __restrict__ sc,
                                                     const Ts* __restrict__ Ls, const Ts* __restrict__ Us,
                                                     const double inv_dx2, const int* __restrict__ done,
@@ -532,50 +537,49 @@ __global__ __launch_bounds__(256) void rowcr_kernel(const BatchPtr<Ts> data, con
     const auto row = as_global(data(blockIdx.y) + (long)k * nx);
     const Ts lk = lmy[lmz ? k / rdiv : k];
     const double lz = lmz ? (double)lmz[k % rdiv] : 0.0;
-    for (int j = threadIdx.x; j < nx; j += blockDim.x) {
-        const T d = lmz ? -2.0 * inv_dx2 - (double)(lk * sc[j]) - lz : -2.0 * inv_dx2 - (double)(lk * sc[j]);
-        const T ej = j > 0 ? (T)(Ls[j] * inv_dx2) : T(0), fj = j < nx - 1 ? (T)(Us[j] * inv_dx2) : T(0);
+    // row j: e x_left - (e + f + s) x + f x_right = b; solved for x (last): x = b +
+    // e x_left + f x_right with s = 1 - e - f
+    auto put = [&](const int j, T ej, T fj, T sj, T b, const bool last) {
+        if (last) {
+            const T inv = T(1) / (ej + fj + sj);
+            ej *= inv;
+            fj *= inv;
+            sj *= inv;
+            b *= -inv;
+        }
         e[j] = ej;
         f[j] = fj;
-        s[j] = (-d - ej) - fj;
-        bb[j] = (T)row[j];
+        s[j] = sj;
+        bb[j] = b;
+    };
+    for (int j = threadIdx.x; j < nx; j += NT) {
+        const T d = lmz ? -2.0 * inv_dx2 - (double)(lk * sc[j]) - lz : -2.0 * inv_dx2 - (double)(lk * sc[j]);
+        const T ej = j > 0 ? (T)(Ls[j] * inv_dx2) : T(0), fj = j < nx - 1 ? (T)(Us[j] * inv_dx2) : T(0);
+        put(j, ej, fj, (-d - ej) - fj, (T)row[j], (j & 1) == 0);
     }
     __syncthreads();
-    auto diag = [&](const int j) { return e[j] + f[j] + s[j]; };
     for (int l = 1; l < q; ++l) {
         const int st = 1 << l, h = st >> 1;
-        for (int j = st - 1 + threadIdx.x * st; j < nx; j += blockDim.x * st) {
-            const T alpha = e[j] / diag(j - h);
-            if (j + h < nx) {
-                const T gamma = f[j] / diag(j + h);
-                s[j] += alpha * s[j - h] + gamma * s[j + h];
-                bb[j] += alpha * bb[j - h] + gamma * bb[j + h];
-                e[j] = alpha * e[j - h];
-                f[j] = gamma * f[j + h];
-            } else {
-                s[j] += alpha * s[j - h];
-                bb[j] += alpha * bb[j - h];
-                e[j] = alpha * e[j - h];
-            }
+        for (int j = st - 1 + threadIdx.x * st; j < nx; j += NT * st) {
+            const bool right = j + h < nx;   // else f[j] is 0
+            const int r = right ? j + h : j;
+            const T ej = e[j], fj = right ? f[j] : T(0);
+            put(j, ej * e[j - h], fj * f[r], s[j] + ej * s[j - h] + fj * s[r], bb[j] - ej * bb[j - h] - fj * bb[r],
+                (j + 1) >> l & 1);
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        const int top = (1 << (q - 1)) - 1;   // <= nx - 1
-        bb[top] = -bb[top] / diag(top);
-    }
-    __syncthreads();
     for (int l = q - 1; l > 0; --l) {
         const int st = 1 << l, h = st >> 1;
-        for (int j = h - 1 + threadIdx.x * st; j < nx; j += blockDim.x * st) {
-            T acc = -bb[j];
-            if (j - h >= 0) acc += e[j] * bb[j - h];
-            if (j + h < nx) acc += f[j] * bb[j + h];
-            bb[j] = acc / diag(j);
+        for (int j = h - 1 + threadIdx.x * st; j < nx; j += NT * st) {
+            T x = bb[j];
+            if (j - h >= 0) x += e[j] * bb[j - h];
+            if (j + h < nx) x += f[j] * bb[j + h];
+            bb[j] = x;
         }
         __syncthreads();
     }
-    for (int j = threadIdx.x; j < nx; j += blockDim.x) row[j] = (Ts)bb[j];
+    for (int j = threadIdx.x; j < nx; j += NT) row[j] = (Ts)bb[j];
 }
 
 // ---------------------------------------------------------------------------
@@ -586,12 +590,13 @@ __global__ __launch_bounds__(256) void rowcr_kernel(const BatchPtr<Ts> data, con
 // terms of the separators left of and in the chunk; the separators' tridiagonal
 // system over the lanes is solved by parallel cyclic reduction (lanes' values by
 // shuffles), and the chunk follows from its two separators.
-// Rows carry their excess s = -d - a - c as in rowcr_kernel.  Error against extended precision, rows of 511 / 1000 points, lowest mode:
-// cyclic reduction 8e-13 / 3e-12, this 1e-15 / 2e-15.  No barrier, and C +
-// log2 of the lanes dependent reciprocals where rowcr_kernel's 2 log2(nx) levels
-// each wait for LDS, a division and a barrier: 511 FP64 rows of 511 points 11.3
-// us there, 5.2 here.  The row is read and written coalesced and turned
-// through LDS (chunk stride C + 1: conflict-free).
+// Rows carry their excess s = -d - a - c as in rowcr_kernel.  Error against an
+// elimination of the same rounded matrix in 60 digits, rows of 511 / 1000 points,
+// lowest mode: cyclic reduction of the diagonals 4e-13 / 2e-12, this 3e-15 / 5e-16.
+// No barrier, and C + log2 of the lanes dependent reciprocals where cyclic
+// reduction's 2 log2(nx) levels each wait for LDS and a barrier: 511 FP64 rows of
+// 511 points 11.3 us there, 5.2 here.  The row is read and written coalesced and
+// turned through LDS (chunk stride C + 1: conflict-free).
 // The arithmetic is FP64 also for FP32 data: the lowest modes' systems are nearly
 // singular (in FP32 the refinement of 511 x 1000 points with a smooth right-hand
 // side stopped at 1.3e-10 after four inner solves).
@@ -902,6 +907,18 @@ static hipError_t rowpart_k(const RowCrArgs& a) {
     return hipGetLastError();
 }
 
+template <typename Ts, int NT>
+static hipError_t rowcr_nt(const RowCrArgs& a, const int q) {
+    const size_t lds = 4 * sizeof(double) * (size_t)a.nx;
+    hipError_t e = allow_lds(rowcr_kernel<Ts, NT>, lds);
+    if (e != hipSuccess) return e;
+    const BatchPtr<Ts> data{(Ts*)a.data, a.data_tab, a.bs};
+    hipLaunchKernelGGL((rowcr_kernel<Ts, NT>), dim3(a.nrows, a.batch), dim3(NT), lds, a.stream, data, a.nx, q,
+                       (const Ts*)a.lmy, (const Ts*)a.sc, (const Ts*)a.Ls, (const Ts*)a.Us, a.inv_dx2, a.done,
+                       (const Ts*)a.lmz, a.rdiv);
+    return hipGetLastError();
+}
+
 template <typename Ts>
 static hipError_t rowcr_k(const RowCrArgs& a) {
     // the fewest unknowns a lane that cover the row; longer rows by LDS
@@ -912,14 +929,11 @@ static hipError_t rowcr_k(const RowCrArgs& a) {
     if (a.nx <= 1024) return rowpart_k<Ts, 16>(a);
     int q = 0;
     while ((1 << q) < a.nx + 1) q++;
-    const size_t lds = 4 * sizeof(double) * (size_t)a.nx;
-    hipError_t e = allow_lds(rowcr_kernel<Ts>, lds);
-    if (e != hipSuccess) return e;
-    const BatchPtr<Ts> data{(Ts*)a.data, a.data_tab, a.bs};
-    hipLaunchKernelGGL((rowcr_kernel<Ts>), dim3(a.nrows, a.batch), dim3(256), lds, a.stream, data, a.nx, q,
-                       (const Ts*)a.lmy, (const Ts*)a.sc, (const Ts*)a.Ls, (const Ts*)a.Us, a.inv_dx2, a.done,
-                       (const Ts*)a.lmz, a.rdiv);
-    return hipGetLastError();
+    // threads a row: as many as keep a CU's wavefronts busy with the rows its LDS
+    // holds, three (up to 1706 points) or two and one (16 x 511 FP64 rows, us a solve with
+    // 256 / 512 / 1024 threads: 1500 points 265 / 240 / 278, 2000 387 / 340 / 326, 4096
+    // 1219 / 974 / 851)
+    return 3 * 4 * sizeof(double) * (size_t)a.nx <= 160 * 1024 ? rowcr_nt<Ts, 512>(a, q) : rowcr_nt<Ts, 1024>(a, q);
 }
 
 template <typename Ts, typename T>
