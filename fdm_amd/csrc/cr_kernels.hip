@@ -233,21 +233,20 @@ __global__ __launch_bounds__((64 * ZcrStripCfg<Q, CR>::G * S)) void zcr_strip_ke
     // all C loads are in flight together
     auto row_at = [&](int r) { return base[(long)(c * C + r < NQ - 1 ? c * C + r : NQ - 2) * plane]; };
     auto put = [&](int r, T x) { v[r] = (valid && c * C + r < NQ - 1) ? x * gamma : T(0); };
-    if constexpr (sizeof(Ts) == sizeof(T)) {
-        // The mode's eigenvalues ahead of the rows: loads return in order, so the
-        // levels are computed while the rows are in flight (31^3 FP64 14.2 -> 13.9 us
-        // a solve, 63^3 20.1 -> 19.9; rows of floats, converted as they come,
-        // measured no faster so).
+    if constexpr (sizeof(Ts) == sizeof(T) || Q == 9) {
+        // as in zcr_kernel; of the rows of floats only at 512 rows, where the levels and
+        // the rows converted to double do not fit the registers together (3 x 127 x 127
+        // x 511: 115 us a launch with the rows converted first, 102 so)
         const T lam = (T)lmx[kx] + (T)lmy[ky];
         __builtin_amdgcn_sched_barrier(0);
-        T raw[C];
+        Ts raw[C];
 #pragma unroll
         for (int r = 0; r < C; ++r) raw[r] = row_at(r);
         __builtin_amdgcn_sched_barrier(0);
         cr_levels<T, Q>(L, b, lam);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int r = 0; r < C; ++r) put(r, raw[r]);
+        for (int r = 0; r < C; ++r) put(r, (T)raw[r]);
     } else {
 #pragma unroll
         for (int r = 0; r < C; ++r) put(r, (T)row_at(r));
