@@ -107,11 +107,20 @@ __device__ __forceinline__ void xtile_sweep(const int xb, const bool on, LD&& ld
     }
 }
 
+// Wavefronts a SIMD the registers are cut for, at most.  FP64 real transforms of 128
+// points fit four, but then few of a tile's loads are in flight: 20 x 128 x 64 x 256
+// points, forward / inverse, us a launch: cut for four 154 / 127, for three 134 / 120.
+template <typename T, int LOGN, int KIND>
+struct XTileWaves {
+    static constexpr int most = sizeof(T) == 8 && LOGN == 7 && KIND != kDst ? 3 : 8;
+};
+
 // rows = nrows pencils of IO::n points (N-1 Dirichlet, N periodic), contiguous;
 // batch via blockIdx.y.  tiles_pp > 0: tiles_pp tiles per plane of rows_pp rows,
 // so a tile's rows (and the pencils that share a transform) lie in one plane.
 template <typename Tin, typename Tout, typename T, int LOGN, bool ACCUM, int KIND, int TILE_>
-__global__ __launch_bounds__((TileCfg<LOGN, T, TILE_>::NT)) void xaxis_dst_kernel(
+__global__ __launch_bounds__((TileCfg<LOGN, T, TILE_>::NT)) __attribute__((amdgpu_waves_per_eu(1, XTileWaves<T, LOGN, KIND>::most)))
+void xaxis_dst_kernel(
     const BatchPtr<const Tin> in, const BatchPtr<Tout> out, const long nrows, const T scale,
     const T* __restrict__ tables, const int* __restrict__ done, int* __restrict__ reset,
     const int tiles_pp, const int rows_pp) {
