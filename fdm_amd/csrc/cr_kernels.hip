@@ -253,17 +253,19 @@ __global__ __launch_bounds__((64 * ZcrStripCfg<Q, CR>::G * S)) void zcr_strip_ke
         cr_levels<T, Q>(L, b, (T)lmx[kx] + (T)lmy[ky]);
     }
 
-    // forward reduction inside the chunk
+    // forward reduction inside the chunk (explicit fma, here and below: the compiler may
+    // else contract the scale of the right-hand side into the first level's sum, in one
+    // kernel and not in another)
     T toRight = T(0), toLeft = T(0);
     static_for<1, LOC + 1>([&](auto ll) {
         constexpr int l = decltype(ll)::value;
         constexpr int st = 1 << l, h = st >> 1;
         const T a = L.alpha[l];
 #pragma unroll
-        for (int r = st - 1; r < C - 1; r += st) v[r] += a * (v[r - h] + v[r + h]);
+        for (int r = st - 1; r < C - 1; r += st) v[r] = fma(a, v[r - h] + v[r + h], v[r]);
         if constexpr (G > 1) {
-            toRight += a * v[C - 1 - h];
-            toLeft += a * v[h - 1];
+            toRight = fma(a, v[C - 1 - h], toRight);
+            toLeft = fma(a, v[h - 1], toLeft);
         }
     });
 
@@ -286,7 +288,7 @@ __global__ __launch_bounds__((64 * ZcrStripCfg<Q, CR>::G * S)) void zcr_strip_ke
             constexpr int st = 1 << lp, h = st >> 1;
             const T a = L.alpha[LOC + lp];
 #pragma unroll
-            for (int i = st - 1; i < G - 1; i += st) sp[i] += a * (sp[i - h] + sp[i + h]);
+            for (int i = st - 1; i < G - 1; i += st) sp[i] = fma(a, sp[i - h] + sp[i + h], sp[i]);
         });
         sp[G / 2 - 1] *= L.inv_d[Q - 1];
         static_for<1, LOGG>([&](auto ll) {
@@ -297,7 +299,7 @@ __global__ __launch_bounds__((64 * ZcrStripCfg<Q, CR>::G * S)) void zcr_strip_ke
             for (int i = h - 1; i < G - 1; i += st) {
                 const T left = i - h >= 0 ? sp[i - h] : T(0);
                 const T right = i + h < G - 1 ? sp[i + h] : T(0);
-                sp[i] = (sp[i] - cc * (left + right)) * id;
+                sp[i] = fma(-cc, left + right, sp[i]) * id;
             }
         });
         T xl = T(0), xr = T(0);
@@ -318,7 +320,7 @@ __global__ __launch_bounds__((64 * ZcrStripCfg<Q, CR>::G * S)) void zcr_strip_ke
 #pragma unroll
         for (int r = h - 1; r < C - 1; r += st) {
             const T left = r - h >= 0 ? v[r - h] : xleft;
-            v[r] = (v[r] - cc * (left + v[r + h])) * id;
+            v[r] = fma(-cc, left + v[r + h], v[r]) * id;
         }
     });
 

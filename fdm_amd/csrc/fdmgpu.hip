@@ -575,15 +575,22 @@ int stage_tridiag(fdmgpu_plan_t* P, void* data, Tab data_tab, int count, hipStre
     return FDMGPU_OK;
 }
 
-// Dirichlet cubes that small_cube_kernel solves in one launch, in the default variant.
-bool use_small_cube(const fdmgpu_plan_t* P) {
+// Dirichlet cubes that small_cube_kernel solves in one launch, in the default
+// variant; the three launches give the same bits.  A FP64 problem of 31 planes keeps
+// its CU longer than the three launches take while these have CUs to spare (one
+// launch / three, us: recorded in a graph 13.8 / 10.5 a problem, 14.4 / 13.0 32 of
+// them, 14.6 / 14.8 48, 14.7 / 17.0 64; a call waited for 28 / 25.7, 28.7 / 28, 28.9 /
+// 30, 29.1 / 32.1).
+constexpr int kSmallCubeBatch31 = 48;
+bool use_small_cube(const fdmgpu_plan_t* P, int count) {
+    if (P->precision == FDMGPU_F64 && P->logz == 5 && count < kSmallCubeBatch31) return false;
     return P->kind == 3 && !P->periodic && P->logx == P->logy && small_cube_ok(P->logx, P->logz) &&
            P->var.plane == 1 && !P->var.tile_x && !P->var.tile_y && !P->var.zcr_gmul;
 }
 
 template <typename T>
 int solve_plain(fdmgpu_plan_t* P, void* ans, Tab ans_tab, const void* rhs, Tab rhs_tab, int count, hipStream_t s) {
-    if (use_small_cube(P)) {
+    if (use_small_cube(P, count)) {
         SmallCubeArgs a{rhs, ans, rhs_tab, ans_tab, plan_elems(P), count, P->dx * std::sqrt(2. / P->lx),
                         P->dy * std::sqrt(2. / P->ly), std::sqrt(2. / P->lx), std::sqrt(2. / P->ly), P->tab_x, P->lmx,
                         P->lmy, 1.0 / (P->hz_op * P->hz_op), zcr_gamma(P), s};

@@ -36,15 +36,28 @@ struct SmallCfg {
 };
 
 // The z system of one mode in one thread (see cr_level in dst_device.hpp), n =
-// 2^Q - 1 rows; v[2^Q - 1] is scratch.
+// 2^Q - 1 rows; v[2^Q - 1] is scratch.  Operation for operation zcr_strip_kernel's in
+// chunks of 16 rows, its default: of 31 rows the middle one separates two chunks,
+// whose parts of its sum are added up apart.  (Explicit fma: else the scale of the
+// right-hand side may be contracted into the first level's sum.)
 template <int Q, typename T>
 __device__ __forceinline__ void cr_column(T (&v)[1 << Q], const CrLevels<T, Q>& L) {
-    constexpr int C = 1 << Q;
+    constexpr int C = 1 << Q, SEP = C > 16 ? C / 2 - 1 : -1;
+    static_assert(C <= 32, "at most two chunks");
+    [[maybe_unused]] T below = T(0), above = T(0);
     static_for<1, Q>([&](auto ll) {
         constexpr int l = decltype(ll)::value, st = 1 << l, h = st >> 1;
 #pragma unroll
-        for (int r = st - 1; r < C - 1; r += st) v[r] += L.alpha[l] * (v[r - h] + v[r + h]);
+        for (int r = st - 1; r < C - 1; r += st) {
+            if (r == SEP) {
+                below = fma(L.alpha[l], v[r - h], below);
+                above = fma(L.alpha[l], v[r + h], above);
+            } else {
+                v[r] = fma(L.alpha[l], v[r - h] + v[r + h], v[r]);
+            }
+        }
     });
+    if constexpr (SEP >= 0) v[SEP] = v[SEP] + below + above;
     v[C / 2 - 1] *= L.inv_d[Q - 1];
     v[C - 1] = T(0);
     static_for<1, Q>([&](auto ll) {
@@ -52,7 +65,7 @@ __device__ __forceinline__ void cr_column(T (&v)[1 << Q], const CrLevels<T, Q>& 
 #pragma unroll
         for (int r = h - 1; r < C - 1; r += st) {
             const T left = r - h >= 0 ? v[r - h >= 0 ? r - h : 0] : T(0);
-            v[r] = (v[r] - L.c[l - 1] * (left + v[r + h])) * L.inv_d[l - 1];
+            v[r] = fma(-L.c[l - 1], left + v[r + h], v[r]) * L.inv_d[l - 1];
         }
     });
 }
