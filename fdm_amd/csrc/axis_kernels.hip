@@ -108,10 +108,11 @@ __device__ __forceinline__ void xtile_sweep(const int xb, const bool on, LD&& ld
 }
 
 // Wavefronts a SIMD the registers are cut for, at most.  FP64 real transforms of 128
-// points fit four, but then few of a tile's loads are in flight: 20 x 128 x 64 x 256
-// points, forward / inverse, us a launch: cut for four 154 / 127, for three 134 / 120.
+// points fit four, but then few of a tile's loads are in flight, us a launch cut for
+// four / three: x, 20 x 128 x 64 x 256 points, forward 154 / 134, inverse 127 / 120;
+// y, 20 x 64 x 128 x 32 points, forward 23.0 / 20.6 (inverse 18.8 / 18.6).
 template <typename T, int LOGN, int KIND>
-struct XTileWaves {
+struct AxisWaves {
     static constexpr int most = sizeof(T) == 8 && LOGN == 7 && KIND != kDst ? 3 : 8;
 };
 
@@ -119,7 +120,7 @@ struct XTileWaves {
 // batch via blockIdx.y.  tiles_pp > 0: tiles_pp tiles per plane of rows_pp rows,
 // so a tile's rows (and the pencils that share a transform) lie in one plane.
 template <typename Tin, typename Tout, typename T, int LOGN, bool ACCUM, int KIND, int TILE_>
-__global__ __launch_bounds__((TileCfg<LOGN, T, TILE_>::NT)) __attribute__((amdgpu_waves_per_eu(1, XTileWaves<T, LOGN, KIND>::most)))
+__global__ __launch_bounds__((TileCfg<LOGN, T, TILE_>::NT)) __attribute__((amdgpu_waves_per_eu(1, AxisWaves<T, LOGN, KIND>::most)))
 void xaxis_dst_kernel(
     const BatchPtr<const Tin> in, const BatchPtr<Tout> out, const long nrows, const T scale,
     const T* __restrict__ tables, const int* __restrict__ done, int* __restrict__ reset,
@@ -213,7 +214,8 @@ constexpr int kAxisXcds = 8;
 // block.  Column p of the tile is stored as LDS row p: the global reads stay
 // row segments of TILE consecutive x, and the transform is the x pass.
 template <typename Tin, typename Tout, typename T, int LOGN, int KIND, int TILE_>
-__global__ __launch_bounds__((TileCfg<LOGN, T, TILE_>::NT)) void yaxis_dst_kernel(
+__global__ __launch_bounds__((TileCfg<LOGN, T, TILE_>::NT)) __attribute__((amdgpu_waves_per_eu(1, AxisWaves<T, LOGN, KIND>::most)))
+void yaxis_dst_kernel(
     const BatchPtr<const Tin> in, const BatchPtr<Tout> out, const int nx, const T scale,
     const T* __restrict__ tables, const int* __restrict__ done, const int nplanes, const int batch,
     int* __restrict__ reset) {
