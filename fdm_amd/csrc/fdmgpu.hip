@@ -306,10 +306,18 @@ namespace {
 constexpr long kPlaneRegPlanes = 192;
 
 // Columns per block of a 2-D plan's y transforms by default: 16, so that the few
-// columns of one problem reach more CUs (one solve in FP64, tiles of 32 / 16 / 64
-// columns, us: 511 x 511 40 / 33 / -, 255 x 255 23 / 20 / 33, 127 x 127 18 / 17 /
-// 22; 50 problems a solve: 192 / 195, 53 / 55, 30 / 30).
-int rect_tile_y(const fdmgpu_plan_t* P) { return P->var.tile_y ? P->var.tile_y : 16; }
+// columns of one problem reach more CUs, except transforms of 32 points, which are
+// too short for it.  The number of problems may not decide: the widths differ in
+// rounding, and a problem's answer does not depend on the batch it is in.
+// Recorded in a graph, tiles of 16 / 32 columns, us a solve of 1 and of 50 problems:
+//   200 x 63    FP32 11.6 / 12.2, 18.6 / 18.8      FP64 11.9 / 12.8, 22.6 / 23.5
+//   200 x 127   FP32 14.9 / 15.8, 32.0 / 32.5      FP64 16.0 / 17.6, 41.2 / 43.2
+//   1000 x 512  FP32 27.0 / 31.5, 187 / 197        FP64 35.4 / 39.0, 350 / 333 (y periodic)
+//   31 x 31     FP32 (FFT2) 15.2 / 14.7, 16.5 / 16.4   FP64 15.5 / 15.7, 17.7 / 18.0
+//   1000 x 31   FP32 12.9 / 12.9, 29.6 / 27.6      FP64 13.1 / 13.3, 40.9 / 37.8
+// 255 points (DST) take half a wavefront to a pair at 16 and pencil_pairs at 32: 511
+// columns FP64 15.2 / 24.0 for one problem, 47.2 / 49.0 for 16, 97 / 91 for 64.
+int rect_tile_y(const fdmgpu_plan_t* P) { return P->var.tile_y ? P->var.tile_y : P->logy == 5 ? 32 : 16; }
 
 bool reg_shape(const fdmgpu_plan_t* P) {
     return P->kind == 3 && P->precision != FDMGPU_F64 && P->logx == 8 && P->logy == 8;
