@@ -7,8 +7,9 @@
 //   (A u)_i = (u_{x-1} - 2u + u_{x+1}) * cx_i  (+ LaplRect scales on x)
 //           + (u_{y-1} - 2u + u_{y+1}) * iy * sy_x
 //           + (u_{z-1} - 2u + u_{z+1}) * iz          (cube only)
-// Norm partials are reduced in a fixed order (no atomics), so a problem's
-// residual and iteration count do not depend on what else is in the batch.
+// Norm partials are stored one by one and summed in a fixed order (atomics only
+// count the blocks that have stored theirs), so a problem's residual and iteration
+// count do not depend on what else is in the batch.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -53,14 +54,18 @@ __device__ __forceinline__ void block_sum2(double& a, double& b, double* sh) {
 // twice its time.)  The storing wave waits until its stores are complete before
 // it counts, so whoever reads the last count reads every partial.
 // Storing, counting and reading back are three round trips past the L2, about
-// 4 us of a block's life.  One round of blocks (kFoldBlocks) hides that at its
-// end; with more rounds each pays it, and a check of its own is cheaper: 50
-// problems of 511 x 71 points, 6400 blocks of four rows, took 467 us a solve
-// folded and 332 apart.
+// 4 us of a block's life.  Beside the columns of planes of a 3-D block that is
+// little while there is one round of blocks (kFoldBlocks); with more rounds each
+// pays it, and a check of its own is cheaper.  A 2-D block has four rows: past a
+// few blocks (fold_2d) the check apart is cheaper, us a solve folded / apart, recorded
+// in a graph: 25 problems of 200 x 15 points (8 blocks each) 56.6 / 58.4, 10 of 50 x
+// 63 (16) 58.0 / 58.0, 16 of them 60.5 / 57.7, one of 50 x 511 (128) 80.1 / 78.1, 6 of
+// them 112 / 89, 16 of 511 x 255 (64) 191 / 165.
 // The counter is the problem's iters[] entry: it enters the launch at `base`
 // (0, or the iteration the problem's previous check wrote) and leaves it as `it`.
 // ---------------------------------------------------------------------------
-constexpr long kFoldBlocks = 1024;   // blocks of a residual launch that checks itself, at most
+constexpr long kFoldBlocks = 1024;   // blocks of a 3-D residual launch that checks itself, at most
+static bool fold_2d(long nblk, int batch) { return nblk * batch <= (nblk <= 32 ? 200 : 64); }
 constexpr int kCheckBlock = 1024;   // threads the summation order is written for
 constexpr int kCheckUnroll = 8;
 
@@ -511,7 +516,7 @@ hipError_t launch_residual(const ResidualArgs& a) {
     } else {
         nblk = residual_partials(a.nx, a.ny, a.nz, false);
         const dim3 grid((unsigned)nblk, a.batch);
-        check.fold = nblk * a.batch <= kFoldBlocks;
+        check.fold = fold_2d(nblk, a.batch);
         if (a.sy)
             hipLaunchKernelGGL((residual_kernel<false, true>), grid, dim3(kResBlock), 0, a.stream, f, u, a.r32,
                                a.partial, a.nx, a.ny, 1, a.ix, a.iy, 0.0, a.sy, a.lx, a.ux, a.bs, skip, check);
