@@ -851,10 +851,13 @@ static hipError_t zcr_g(const ZcrArgs& a) {
     // default: Dirichlet systems in the strip layout (64 consecutive modes per
     // wave) with 16-row chunks up to 128 rows (measured fastest at 128 rows:
     // 8 waves per SIMD in FP32) and 32-row chunks from 256 rows (measured 2-3%
-    // faster than 16 at 256 rows, FP64 and FP32); circulant ones with 2 lanes
-    // per 64 rows from 64 rows up (fewer registers per lane, twice the
-    // occupancy of 1)
+    // faster than 16 at 256 rows, FP64 and FP32), except the double elimination of
+    // 512 rows of floats, which spills in strips (FP32 solves of 127 x 127 x 511 points,
+    // us, strips / 1: one 84.9 / 72.7, 3 212 / 160, 5 397 / 254; 255 x 255 x 511 344 / 305);
+    // circulant ones with 2 lanes per 64 rows from 64 rows up (fewer registers per
+    // lane, twice the occupancy of 1)
     const int gm = a.gmul                                             ? a.gmul
+                   : (!a.periodic && Q == 9 && sizeof(Ts) < sizeof(T)) ? 1
                    : (!a.periodic && Q <= 7 && zcr_gmul_ok(Q, 5)) ? 5
                    : (!a.periodic && zcr_gmul_ok(Q, 3))           ? 3
                    : (!a.periodic && zcr_gmul_ok(Q, 5))           ? 5

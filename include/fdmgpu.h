@@ -158,7 +158,8 @@ int fdmgpu_solve_batch_noalloc(fdmgpu_plan plan, int count, void* d_ans, const v
  * wavefront per 32-row chunk of 64 consecutive modes, 64 (3) or 128 (4)
  * modes per block (Dirichlet z, 32 to 512 rows; 4 up to 128), 5 = the same
  * with 16-row chunks (16 to 256 rows); 0 = default
- * (Dirichlet: 5 up to 128 rows, 3 from 256 rows, else 5 where valid;
+ * (Dirichlet: 5 up to 128 rows, 3 from 256 rows (LaplCube<float>: 1 at 512),
+ * else 5 where valid;
  * circulant: 2 from 64 rows, else 1); tile_y = 0 takes 64 for a cube's FP32
  * planes at least 128 wide when two such blocks fit a CU, else 32 (16 where 32
  * does not fit), and 16 for 2-D plans (32 where y transforms have 32 points); fuse (FP32+refine plane path) = FP64 residual fused into the next
