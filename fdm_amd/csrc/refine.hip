@@ -60,11 +60,16 @@ __device__ __forceinline__ void block_sum2(double& a, double& b, double* sh) {
 // few blocks (fold_2d) the check apart is cheaper, us a solve folded / apart, recorded
 // in a graph: 25 problems of 200 x 15 points (8 blocks each) 56.6 / 58.4, 10 of 50 x
 // 63 (16) 58.0 / 58.0, 16 of them 60.5 / 57.7, one of 50 x 511 (128) 80.1 / 78.1, 6 of
-// them 112 / 89, 16 of 511 x 255 (64) 191 / 165.
+// them 112 / 89, 16 of 511 x 255 (64) 191 / 165.  The check after the fourth solve finds
+// every problem done as a rule, and the blocks of such end before they store or
+// count: there the launch saved is worth more whatever the size (50 problems of 200 x
+// 63 points 84.5 -> 83.0; after the third solve too 81.3, but problems that need it pay:
+// 6 of 50 x 511 points 87.7 -> 95.7).
 // The counter is the problem's iters[] entry: it enters the launch at `base`
 // (0, or the iteration the problem's previous check wrote) and leaves it as `it`.
 // ---------------------------------------------------------------------------
 constexpr long kFoldBlocks = 1024;   // blocks of a 3-D residual launch that checks itself, at most
+constexpr int kFoldFrom = 4;         // or after this inner solve, whatever its size
 static bool fold_2d(long nblk, int batch) { return nblk * batch <= (nblk <= 32 ? 200 : 64); }
 constexpr int kCheckBlock = 1024;   // threads the summation order is written for
 constexpr int kCheckUnroll = 8;
@@ -463,7 +468,7 @@ static void launch_residual_tile(const ResidualArgs& a, const BatchPtr<const dou
     // the kernel re-deals the blocks (problem, chunk, tile) to XCD slabs
     const long total = (long)tiles * zc * a.batch;
     const dim3 grid((unsigned)((total + kXcdCount - 1) / kXcdCount * kXcdCount));
-    check.fold = total <= kFoldBlocks;
+    check.fold = total <= kFoldBlocks || a.it >= kFoldFrom;
     if (a.r32)
         hipLaunchKernelGGL((residual_tile_kernel<TX, TY, true, Tu>), grid, dim3(TX * TY), 0, a.stream, f, u, a.r32,
                            a.partial, a.nx, a.ny, a.nz, a.ix, a.iy, a.iz, a.bs, a.batch, cg,
@@ -516,7 +521,7 @@ hipError_t launch_residual(const ResidualArgs& a) {
     } else {
         nblk = residual_partials(a.nx, a.ny, a.nz, false);
         const dim3 grid((unsigned)nblk, a.batch);
-        check.fold = fold_2d(nblk, a.batch);
+        check.fold = fold_2d(nblk, a.batch) || a.it >= kFoldFrom;
         if (a.sy)
             hipLaunchKernelGGL((residual_kernel<false, true>), grid, dim3(kResBlock), 0, a.stream, f, u, a.r32,
                                a.partial, a.nx, a.ny, 1, a.ix, a.iy, 0.0, a.sy, a.lx, a.ux, a.bs, skip, check);
