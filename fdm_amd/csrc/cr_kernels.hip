@@ -156,9 +156,10 @@ __global__ __launch_bounds__(256) void zcr_kernel(const BatchPtr<Ts> data, const
     auto put = [&](int r, T x) { v[r] = (valid && c * C + r < NQ - 1) ? x * gamma : T(0); };
     if constexpr (sizeof(Ts) == sizeof(T)) {
         // The mode's eigenvalues ahead of the rows: loads return in order, so the
-        // levels are computed while the rows are in flight (31^3 FP64 14.2 -> 13.9 us
-        // a solve, 63^3 20.1 -> 19.9; rows of floats, converted as they come,
-        // measured no faster so).
+        // levels are computed while the rows are in flight (FP64 solves recorded in a
+        // graph, with the levels of the diagonals after the rows / this: 31^3 13.2 / 13.0
+        // us, 63^3 20.0 / 19.8; rows of floats, converted as they come, measured no
+        // faster so).
         const T lam = (T)lmx[kx] + (T)lmy[ky];
         __builtin_amdgcn_sched_barrier(0);
         T raw[C];

@@ -937,8 +937,11 @@ struct WaveDst {
 //
 // Layout: rows of pitch P = 129, no swizzle; a job takes pencils q and q + 1, the
 // two jobs of 32 lanes pencils 16 apart.  In every access a job's 16 lanes take
-// slots distinct mod 16, and 16 rows or columns are 16 banks mod 32, so reads
-// (32 lanes) and writes (16 of eight bytes) are free of conflicts in both passes.
+// slots distinct mod 16, and 16 rows or columns are 16 banks mod 32: by banks of
+// eight bytes no read of 32 lanes or write of 16 meets a conflict.  The counters
+// show 0.25 conflict cycles an LDS instruction in the streaming kernel, staging and
+// store phase included, where the 8-lane form's skewed layout had 0.14: what the
+// form gains it gains by the wavefronts.
 // Slots: exchange 1 at 16 k2 + (t ^ 2 k2); Z by posZ (bits 4, 5 of k into bits
 // 0, 1, bit 6 into bit 3), where the periodic kinds leave their outputs; DST
 // outputs by sigma, as DstShape<7>.

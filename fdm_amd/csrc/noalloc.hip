@@ -10,8 +10,9 @@
 // hipGetSymbolAddress and kept in g_scratch[device].  Every call on one GPU
 // shares that GPU's array (calls that overlap on one GPU race: the caller
 // orders them, e.g. on one stream), and it keeps the previous call's
-// contents; what must start at zero (the per-problem convergence flags and
-// iteration counts) is cleared by a fill kernel at the start of every solve.
+// contents: the per-problem iteration counts are cleared by a solve's first
+// transform (or a fill kernel), and the first check sets the convergence flags
+// without reading them.
 #include <hip/hip_runtime.h>
 
 #include <cstdio>

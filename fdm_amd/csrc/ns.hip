@@ -523,7 +523,9 @@ int fdmgpu_ns_step(fdmgpu_ns N, int count, void* stream) {
     // time than all but the smallest grids' steps run; steps behind others hide
     // even that.  Replayed / one by one, us a step: 127^3 FP32+refine 194 / 188,
     // FP64 127 / 121; 31^3 FP64 40 / 30 in calls of ten steps, 59 / 67 in calls of one;
-    // 63^3 FP64 in calls of one 69 / 64.
+    // 63^3 FP64 in calls of one 69 / 64; 31^3 FP32+refine in calls of ten 92 / 85, in
+    // calls of one 114 / 106, 15^3 90 / 82 and 108 / 100.  The calling thread pays for it
+    // in long calls: 25 us a step instead of 19 (FP64), 37 instead of 26 (FP32+refine).
     const bool replay = count == 1 && N->plan->precision == FDMGPU_F64 &&
                         (long)N->g.nx * N->g.ny * N->g.nz <= kReplayPoints;
     for (int c = 0; c < count; c++) {

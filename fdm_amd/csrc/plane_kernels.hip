@@ -193,7 +193,9 @@ __attribute__((amdgpu_waves_per_eu(PlaneCfg<LOGN>::template waves<T>()))) void p
 // measured with s_memtime stamps.)  Both passes are wide_pairs128's, in its
 // layout; results agree with plane_dst_kernel's to FP64 rounding (2e-14
 // relative at 127^3), not bitwise.  What bounds it: a launch of 32 x 127 planes
-// takes about 250 us, its 1.05 GB at the rate of a large copy 213.
+// takes about 240 us by events around the launches of a solve (303 in a kernel
+// trace, which slows this kernel by a fifth), its 1.05 GB at the rate of a large
+// copy (4.95 TB/s) 212 and at that of the z systems' kernel (5.75) 182.
 // ---------------------------------------------------------------------------
 struct StreamCfg {
     static constexpr int N = 128, NT = 1024, P = kWidePitch;

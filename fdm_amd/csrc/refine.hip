@@ -46,7 +46,11 @@ __device__ __forceinline__ void block_sum2(double& a, double& b, double* sh) {
 // after every residual, 9 us at 255^3, and needed a launch that cleared the
 // flags first.  With the fold a residual launch ends about 5 us later and five
 // launches of a solve are gone: 255^3 526 -> 507 us a solve, 32 x 127^3 1320 ->
-// 1310, 512 uneven problems 3797 -> 3680, a 127^3 cavity step 203 -> 199.
+// 1310, 512 uneven problems 3797 -> 3680, a 127^3 cavity step 203 -> 199, 31^3 64.5 ->
+// 60 recorded in a graph.  Where launches are few and long it gains nothing (32 x
+// 127^3 with two inner solves allowed: norm-only residual 0.228 ms before and now),
+// and summing a granule's waves in the loop, for fewer partials to read back, costs
+// the smallest tiles: 300 x 15 x 15 x 31 143 -> 148.
 // What makes the fold cheap is that no release fence is needed: the partials
 // are the only data handed over, and they are stored and loaded as agent-scope
 // atomics, which go past the XCD's L2 by themselves.  (A release at agent scope
